@@ -1980,10 +1980,13 @@ __device__ __forceinline__ void gemm_load_xs(__amdgpu_buffer_rsrc_t xr, uint32_t
     for (int k = 0; k < 4; k++) {
         const int f = QT == FH3K_Q6_K ? 16 * (s >> 2) + 8 * ((s >> 1) & 1) + 2 * (s & 1) + (k & 1) + 4 * (k >> 1)
                                       : s * 4 + k;
-        const int so = f * 1024;
+        // TBW = 1: xf[a][2p + u] is half u (16 tokens) of the fragment pair p,
+        // whose fragments 2p and 2p + 1 are neighbours for every type
+        const int so = TBW == 1 ? (f - (k & 1)) * 1024 : f * 1024;
+        const int lo = TBW == 1 ? (int)xoff + 256 * (k & 1) : (int)xoff;
 #pragma unroll
         for (int a = 0; a < TBW; a++)
-            xf[a][k] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)xoff, so + a * tbs, 0));
+            xf[a][k] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(xr, lo, so + a * tbs, 0));
     }
 }
 
@@ -1995,19 +1998,50 @@ __device__ __forceinline__ void gemm_load_x(const half8 *xa0, const half8 *xa1, 
     }
 }
 
+// Lane l of a 16x16x32 operand holds row l % 16 at k offset 8 * (l / 16): in
+// a pair of 32-row x 16-k fragments (k 0..15, 16..31) that is 16-byte slot
+// 64 * (l / 32) + 32 * ((l / 16) % 2) + l % 16, + 16 for the rows' upper half.
+__device__ __forceinline__ int frag32_slot(int lane) {
+    return 64 * (lane >> 5) + 32 * ((lane >> 4) & 1) + (lane & 15);
+}
+
+// The MFMA and with it the accumulators of a wavefront: one token block runs
+// v_mfma_f32_16x16x32_f16 (2 x 8 blocks of 16x16), two run
+// v_mfma_f32_32x32x16_f16 (2 x 4 blocks of 32x32).  The 16x16 form reads and
+// writes half the accumulator registers per product and draws less power, and
+// gives the same bits; 300 tokens, K = 5120, N = 17408: 91.6 -> 84.8 us per
+// call.  With two token blocks its shorter slots left no room for the
+// dequantisation (100 registers spilled).
+template <int TBW> struct GemmAcc { f32x4 v[2][8]; };
+template <> struct GemmAcc<2> { f32x16 v[2][4]; };
+
 template <int TBW>
-__device__ __forceinline__ void gemm_mfma(half8 (*ldsb)[64], int lane, const half8 (&xf)[TBW][4],
-                                          f32x16 (&acc)[TBW][4]) {
+__device__ __forceinline__ void gemm_mfma(const half8 (*ldsb)[64], int slot, const half8 (&xf)[TBW][4],
+                                          GemmAcc<TBW> &acc) {
+    if constexpr (TBW == 1) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        half8 bfr[4];
+        for (int k = 0; k < 2; k++) {
+            half8 bfr[8];
 #pragma unroll
-        for (int ob = 0; ob < 4; ob++) bfr[ob] = ldsb[ob * 4 + k][lane];
+            for (int ob = 0; ob < 8; ob++) bfr[ob] = (&ldsb[(ob >> 1) * 4 + 2 * k][0])[slot + 16 * (ob & 1)];
 #pragma unroll
-        for (int ob = 0; ob < 4; ob++)
+            for (int ob = 0; ob < 8; ob++)
 #pragma unroll
-            for (int a = 0; a < TBW; a++)
-                acc[a][ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[a][k], bfr[ob], acc[a][ob], 0, 0, 0);
+                for (int u = 0; u < 2; u++)
+                    acc.v[u][ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[0][2 * k + u], bfr[ob], acc.v[u][ob], 0, 0, 0);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            half8 bfr[4];
+#pragma unroll
+            for (int ob = 0; ob < 4; ob++) bfr[ob] = ldsb[ob * 4 + k][slot];
+#pragma unroll
+            for (int ob = 0; ob < 4; ob++)
+#pragma unroll
+                for (int a = 0; a < TBW; a++)
+                    acc.v[a][ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[a][k], bfr[ob], acc.v[a][ob], 0, 0, 0);
+        }
     }
 }
 
@@ -2020,25 +2054,25 @@ __device__ __forceinline__ void gemm_mfma(half8 (*ldsb)[64], int lane, const hal
 // per three MFMAs and the LDS writes after MFMA 20 (the best of a sweep of
 // these counts on the DiT shapes).  Without it the compiler clusters the
 // loads and the dequant into runs that stall the matrix pipe.
-// With one token block per wavefront (TBW = 1: 16 MFMAs and 6 loads per step)
-// the same pattern is compressed: eight VALU per MFMA, the 12 remaining
-// B-fragment reads on three of every four MFMAs, a load every third MFMA and
-// the LDS writes after MFMA 10.
+// With one token block per wavefront (TBW = 1: 32 MFMAs of half the length
+// and 6 loads per step) the same pattern in half-length slots: four VALU per
+// MFMA, the eight B-fragment reads of the second half on every second MFMA, a
+// load every sixth and the LDS writes after MFMA 20.
 template <int TBW, int I>
 __device__ __forceinline__ void gemm_pipe_slot() {
-    constexpr int NM = 16 * TBW;
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);               // MFMA
-    __builtin_amdgcn_sched_group_barrier(0x002, 128 / NM, 0);        // VALU
-    if constexpr (TBW == 2 ? (I % 2 == 1 && I < 24) : (I % 4 != 0))  // DS read
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+    __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+    if constexpr (TBW == 2 ? (I % 2 == 1 && I < 24) : (I % 2 == 1 && I < 16))  // DS read
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    if constexpr (I % 3 == 0 && I < 3 * (2 + 4 * TBW)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
-    if constexpr (I >= 10 * TBW && I < 10 * TBW + 4) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // DS write
-    if constexpr (I + 1 < NM) gemm_pipe_slot<TBW, I + 1>();
+    if constexpr (TBW == 2 ? (I % 3 == 0 && I < 30) : (I % 6 == 0 && I < 36))  // VMEM read
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    if constexpr (I >= 20 && I < 24) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // DS write
+    if constexpr (I + 1 < 32) gemm_pipe_slot<TBW, I + 1>();
 }
 
 template <int TBW>
 __device__ __forceinline__ void gemm_pipe() {
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // B fragments of the first k-slice
+    __builtin_amdgcn_sched_group_barrier(0x100, TBW == 2 ? 4 : 8, 0);  // B fragments of the first k-slice
     gemm_pipe_slot<TBW, 0>();
 }
 
@@ -2093,17 +2127,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
     const int tbs = kf_n * 1024;
     const __amdgpu_buffer_rsrc_t xr =
         buf_rsrc(X16 + ((size_t)(m0 / 32 + TBW * wave) * kf_n) * 64, (uint32_t)TBW * (uint32_t)tbs);
-    const uint32_t xoff = (uint32_t)lane * 16u;
+    const int fslot = TBW == 1 ? frag32_slot(lane) : lane;
+    const uint32_t xoff = (uint32_t)fslot * 16u;
 
     // super-blocks [sb0, sb1) of K: all of them, or this workgroup's window
     const int nsb = K / 256;
     const int sb0 = ks * C;
     const int sb1 = sb0 + C < nsb ? sb0 + C : nsb;
-    f32x16 acc[TBW][4];
-#pragma unroll
-    for (int a = 0; a < TBW; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = f32x16{};
+    GemmAcc<TBW> acc = {};
 
     GemmRaw<QT> re, ro;              // raw weights of even / odd steps
     half8 xe[TBW][4], xo[TBW][4];  // activations of even / odd steps
@@ -2124,7 +2155,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         gemm_load_raw<QT, 2>(wr, wbase, woff, woffq, sb, re, ro);
         gemm_dequant<QT, 1>(lds[1], ro, wf, wl, h);
         __builtin_amdgcn_s_setprio(2);
-        gemm_mfma(lds[0], lane, xe, acc);
+        gemm_mfma<TBW>(lds[0], fslot, xe, acc);
         gemm_pipe<TBW>();
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
@@ -2133,7 +2164,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         gemm_load_raw<QT, 3>(wr, wbase, woff, woffq, sb, ro, re);
         gemm_dequant<QT, 2>(lds[0], re, wf, wl, h);
         __builtin_amdgcn_s_setprio(2);
-        gemm_mfma(lds[1], lane, xo, acc);
+        gemm_mfma<TBW>(lds[1], fslot, xo, acc);
         gemm_pipe<TBW>();
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
@@ -2142,7 +2173,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         gemm_load_raw<QT, 0>(wr, wbase, woff, woffq, nb, re, ro);
         gemm_dequant<QT, 3>(lds[1], ro, wf, wl, h);
         __builtin_amdgcn_s_setprio(2);
-        gemm_mfma(lds[0], lane, xe, acc);
+        gemm_mfma<TBW>(lds[0], fslot, xe, acc);
         gemm_pipe<TBW>();
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
@@ -2151,14 +2182,20 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         gemm_load_raw<QT, 1>(wr, wbase, woff, woffq, nb, ro, re);
         gemm_dequant<QT, 0>(lds[0], re, wf, wl, h);
         __builtin_amdgcn_s_setprio(2);
-        gemm_mfma(lds[1], lane, xo, acc);
+        gemm_mfma<TBW>(lds[1], fslot, xo, acc);
         gemm_pipe<TBW>();
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
     }
 
-    // epilogue: 32x32 output D, lane l holds column l%32 (weight row) and rows
-    // 8*(v/4) + 4*(l/32) + v%4 (tokens).
+    // epilogue by 32x32 output blocks, 16 values per lane: value v is column
+    // (weight row) vcol(v) and row (token) vrow(v) of the block
+    auto vrow = [&](int v) { return TBW == 1 ? 16 * (v >> 3) + 4 * (lane >> 4) + (v & 3) : 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3); };
+    auto vcol = [&](int v) { return TBW == 1 ? 16 * ((v >> 2) & 1) + (lane & 15) : lane & 31; };
+    auto vacc = [&](int tb, int ob, int v) {
+        if constexpr (TBW == 1) return acc.v[v >> 3][2 * ob + ((v >> 2) & 1)][v & 3];
+        else return acc.v[tb][ob][v];
+    };
     // Fast path: a 32x32 block whose rows and 32 columns are all inside the
     // output (row stride a multiple of 4 floats) goes through this wavefront's
     // 4 KiB of LDS (free after the loop's last barrier) and leaves as 16-byte
@@ -2170,7 +2207,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
     // mode 0 store, 1 gate residual (dst += g * y, g at the same offsets in aux)
     auto block_store = [&](const float (&val)[16], float *dst, const float *g, size_t ld, int mode) {
 #pragma unroll
-        for (int v = 0; v < 16; v++) stg[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * 32 + (lane & 31)] = val[v];
+        for (int v = 0; v < 16; v++) stg[vrow(v) * 32 + vcol(v)] = val[v];
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -2207,7 +2244,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
                                                      : n0 + 32 * ob;
                     float vals[16];
 #pragma unroll
-                    for (int v = 0; v < 16; v++) vals[v] = acc[tb][ob][v];
+                    for (int v = 0; v < 16; v++) vals[v] = vacc(tb, ob, v);
                     block_store(vals, part + ((size_t)ks * M + tb0) * N + c0, nullptr, (size_t)N, 0);
                 }
             }
@@ -2215,17 +2252,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         }
 #pragma unroll
         for (int tb = 0; tb < TBW; tb++) {
-            const int tbase = wt0 + 32 * tb + 4 * (lane >> 5);
 #pragma unroll
             for (int ob = 0; ob < 4; ob++) {
-                int o = n0 + 32 * ob + (lane & 31);
-                if (epi == EPI_SWIGLU) o = ob < 2 ? nt * 64 + 32 * ob + (lane & 31) : F + nt * 64 + 32 * (ob - 2) + (lane & 31);
-                if (o >= N) continue;
-                float *pp = part + (size_t)ks * M * N + o;
+                const int c0 = epi == EPI_SWIGLU ? (ob < 2 ? nt * 64 + 32 * ob : F + nt * 64 + 32 * (ob - 2)) : n0 + 32 * ob;
+                float *pp = part + (size_t)ks * M * N;
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    const int t = tbase + 8 * (v >> 2) + (v & 3);
-                    if (t < M) pp[(size_t)t * N] = acc[tb][ob][v];
+                    const int t = wt0 + 32 * tb + vrow(v), o = c0 + vcol(v);
+                    if (t < M && o < N) pp[(size_t)t * N + o] = vacc(tb, ob, v);
                 }
             }
         }
@@ -2240,13 +2274,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
                 const int tb0 = wt0 + 32 * tb;
 #pragma unroll
                 for (int ob = 0; ob < 2; ob++) {
-                    const int o = nt * 64 + 32 * ob + (lane & 31);
-                    const float bv = bias ? bias[o] : 0.f, bg = bias ? bias[F + o] : 0.f;
                     float vals[16];
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const int t = tb0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                        vals[v] = (acc[tb][ob][v] * xs_inv[t] + bv) * silu_f32(acc[tb][ob + 2][v] * xs_inv[t] + bg);
+                        const int t = tb0 + vrow(v), o = nt * 64 + 32 * ob + vcol(v);
+                        const float bv = bias ? bias[o] : 0.f, bg = bias ? bias[F + o] : 0.f;
+                        vals[v] = (vacc(tb, ob, v) * xs_inv[t] + bv) * silu_f32(vacc(tb, ob + 2, v) * xs_inv[t] + bg);
                     }
                     block_store(vals, Y + (size_t)tb0 * F + nt * 64 + 32 * ob, nullptr, (size_t)F, 0);
                 }
@@ -2255,17 +2288,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         }
 #pragma unroll
         for (int tb = 0; tb < TBW; tb++) {
-            const int tbase = wt0 + 32 * tb + 4 * (lane >> 5);
 #pragma unroll
             for (int ob = 0; ob < 2; ob++) {
-                const int o = nt * 64 + 32 * ob + (lane & 31);
-                const float bv = bias ? bias[o] : 0.f, bg = bias ? bias[F + o] : 0.f;
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    const int t = tbase + 8 * (v >> 2) + (v & 3);
+                    const int t = wt0 + 32 * tb + vrow(v), o = nt * 64 + 32 * ob + vcol(v);
+                    const float bv = bias ? bias[o] : 0.f, bg = bias ? bias[F + o] : 0.f;
                     if (t < M)
-                        Y[(size_t)t * F + o] = (acc[tb][ob][v] * xs_inv[t] + bv) *
-                                               silu_f32(acc[tb][ob + 2][v] * xs_inv[t] + bg);
+                        Y[(size_t)t * F + o] = (vacc(tb, ob, v) * xs_inv[t] + bv) *
+                                               silu_f32(vacc(tb, ob + 2, v) * xs_inv[t] + bg);
                 }
             }
         }
@@ -2277,12 +2308,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
             const int tb0 = wt0 + 32 * tb;
 #pragma unroll
             for (int ob = 0; ob < 4; ob++) {
-                const int o = n0 + 32 * ob + (lane & 31);
-                const float bo = bias ? bias[o] : 0.f;
                 float vals[16];
 #pragma unroll
                 for (int v = 0; v < 16; v++)
-                    vals[v] = acc[tb][ob][v] * xs_inv[tb0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)] + bo;
+                    vals[v] = vacc(tb, ob, v) * xs_inv[tb0 + vrow(v)] + (bias ? bias[n0 + 32 * ob + vcol(v)] : 0.f);
                 const size_t off = (size_t)tb0 * N + n0 + 32 * ob;
                 block_store(vals, Y + off, epi == EPI_GATE_RES ? aux + off : nullptr, (size_t)N,
                             epi == EPI_GATE_RES ? 1 : 0);
@@ -2292,16 +2321,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
     }
 #pragma unroll
     for (int tb = 0; tb < TBW; tb++) {
-        const int tbase = wt0 + 32 * tb + 4 * (lane >> 5);
 #pragma unroll
         for (int ob = 0; ob < 4; ob++) {
-            const int o = n0 + 32 * ob + (lane & 31);
-            if (o >= N) continue;
-            const float bo = bias ? bias[o] : 0.f;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const int t = tbase + 8 * (v >> 2) + (v & 3);
-                if (t < M) epi_store(Y, aux, epi, (size_t)t * N + o, acc[tb][ob][v] * xs_inv[t] + bo);
+                const int t = wt0 + 32 * tb + vrow(v), o = n0 + 32 * ob + vcol(v);
+                if (t < M && o < N)
+                    epi_store(Y, aux, epi, (size_t)t * N + o, vacc(tb, ob, v) * xs_inv[t] + (bias ? bias[o] : 0.f));
             }
         }
     }
@@ -2490,6 +2516,21 @@ __global__ __launch_bounds__(512) void k_skinny16(const _Float16 *__restrict__ W
     }
 }
 
+__device__ __forceinline__ void gemm16_mfma(half8 (*ldsb)[64], int lane, const half8 (&xf)[2][4],
+                                            f32x16 (&acc)[2][4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        half8 bfr[4];
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++) bfr[ob] = ldsb[ob * 4 + k][lane];
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++)
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+                acc[a][ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[a][k], bfr[ob], acc[a][ob], 0, 0, 0);
+    }
+}
+
 // Large M on fp16 rows: the k_gemm tile (256 tokens x 128 rows, 4 wavefronts
 // of 64 tokens, v_mfma_f32_32x32x16_f16) with the B fragments copied from W16
 // instead of dequantised: per K step of 64, thread (r, h) moves k 16h..16h+15
@@ -2537,7 +2578,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm16(const _Float16 *__restrict__ 
             wb[0] = p[0], wb[1] = p[1], wb[2] = p[4], wb[3] = p[5];
             gemm_load_x(xa0, xa1, s + 1, xn);
         }
-        gemm_mfma(lds[cur], lane, xc, acc);
+        gemm16_mfma(lds[cur], lane, xc, acc);
         if (more) {
             lds[cur ^ 1][wf + h][wl] = wb[0], lds[cur ^ 1][wf + h][wl + 32] = wb[1];
             lds[cur ^ 1][wf + 2 + h][wl] = wb[2], lds[cur ^ 1][wf + 2 + h][wl + 32] = wb[3];
