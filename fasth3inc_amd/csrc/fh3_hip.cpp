@@ -33,6 +33,8 @@ struct State {
     DevBuf ws;                      // x16 fragments + per-row scales
     DevBuf ws2;                     // x16 made from a prepared fp32 copy (other weight types)
     DevBuf w16;                     // fp16 rows of a weight of another type
+    DevBuf wfrag;                   // fp16 fragments of a large product's weights (wfrag_take)
+    hipEvent_t wfrag_used = nullptr;  // after the last product that read wfrag
     DevBuf part;                    // split-K partial sums of the middle-M kernel
     DevBuf attn;                    // fp16 attention operands (Qp, Kp, Vt)
     DevBuf vsa_ws;                  // VSA operands, tile statistics, scores and tile lists
@@ -131,6 +133,49 @@ int grow(DevBuf &b, size_t need, hipStream_t st) {
     FH3_HIPCALL(hipMalloc(&b.p, need));
     b.cap = need;
     return FH3_OK;
+}
+
+// The large products' weight fragments, for one product on `st` (g.mu held;
+// wfrag_release after its launches).  One buffer serves every stream: each user
+// waits on the device for the one before it, so products on different
+// streams stay safe, as they were when k_gemm needed no such memory.  NULL -- the
+// product then reads its weights in place (k_gemm, the same bits) -- when the
+// stream is being captured (a graph must not hold the shared buffer or wait
+// for events outside it) or the memory is not to be had.
+void *wfrag_take(size_t bytes, hipStream_t st) {
+    if (capturing(st)) return nullptr;
+    if (!g.wfrag_used && hipEventCreateWithFlags(&g.wfrag_used, hipEventDisableTiming) != hipSuccess) {
+        g.wfrag_used = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (g.wfrag.cap < bytes) {
+        // allocate and free without disturbing another thread's capture
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (g.wfrag.p) {
+            (void)hipEventSynchronize(g.wfrag_used);
+            (void)hipFree(g.wfrag.p);
+        }
+        g.wfrag = DevBuf();
+        const hipError_t e = hipMalloc(&g.wfrag.p, bytes);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess) {
+            g.wfrag.p = nullptr;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        g.wfrag.cap = bytes;
+    } else if (hipStreamWaitEvent(st, g.wfrag_used, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return g.wfrag.p;
+}
+
+hipError_t wfrag_release(hipStream_t st) {
+    const hipError_t e = hipEventRecord(g.wfrag_used, st);
+    return e == hipSuccess ? e : hipStreamSynchronize(st);
 }
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
@@ -294,13 +339,15 @@ extern "C" void fh3_hip_shutdown(void) {
     std::lock_guard<std::recursive_mutex> lk(g.mu);
     if (!g.init) return;
     (void)hipDeviceSynchronize();
-    DevBuf *bufs[] = {&g.ws, &g.ws2, &g.w16, &g.part, &g.attn, &g.vsa_ws, &g.vsa_geo,
+    DevBuf *bufs[] = {&g.ws, &g.ws2, &g.w16, &g.wfrag, &g.part, &g.attn, &g.vsa_ws, &g.vsa_geo,
                       &g.st_w, &g.st_x, &g.st_y, &g.st_b};
     for (DevBuf *b : bufs) {
         if (b->p) (void)hipFree(b->p);
         b->p = nullptr;
         b->cap = 0;
     }
+    if (g.wfrag_used) (void)hipEventDestroy(g.wfrag_used);
+    g.wfrag_used = nullptr;
     for (auto &r : g.regs) (void)hipFree(r.dev);
     g.regs.clear();
     for (void *p : g.retired) (void)hipFree(p);
@@ -576,12 +623,35 @@ static size_t part16_bytes(const Fh3W *w, int n_tok) {
     return fh3k_gemm_part_bytes(N, K, n_tok, FH3_EPI_NONE);
 }
 
+// The product of k_gemm's path through decoded fragments, where that is the
+// faster form: `done` says whether it was taken.  Called with g.mu held.
+static int product_wfrag(const Fh3W *w, const void *x16, const float *xs_inv, int n_tok, const float *bias, float *d_y,
+                         int epi, const float *aux, hipStream_t st, bool *done) {
+    *done = false;
+    const int K = (int)w->in, N = (int)w->out;
+    const size_t wb = fh3k_gemm256_bytes(w->type, N, K, n_tok, epi);
+    void *wf = wb ? wfrag_take(wb, st) : nullptr;
+    if (!wf) return FH3_OK;
+    *done = true;
+    const hipError_t e = fh3k_gemm256(w->type, w->data, (int64_t)fh3_row_bytes(w->type, w->in), N, K, x16, xs_inv, bias,
+                                      d_y, n_tok, epi, aux, wf, st);
+    const hipError_t r = wfrag_release(st);
+    FH3_HIPCALL(e);
+    FH3_HIPCALL(r);
+    return FH3_OK;
+}
+
 // Called with g.mu held (it may grow the library's buffers).
 static int product16(const Fh3W *w, const void *x16, const float *xs_inv, int n_tok, const float *bias, float *d_y,
                      hipStream_t st) {
     const int K = (int)w->in, Kp = (int)kpad(w->in), N = (int)w->out;
     if (reads_in_place_q(w, n_tok)) {
         const int64_t rb = (int64_t)fh3_row_bytes(w->type, w->in);
+        if (path16(n_tok, w->in) != FH3_HIP_PATH_SKINNY) {
+            bool done;
+            int rc = product_wfrag(w, x16, xs_inv, n_tok, bias, d_y, FH3_EPI_NONE, nullptr, st, &done);
+            if (rc != FH3_OK || done) return rc;
+        }
         float *part = nullptr;
         if (const size_t pb = part16_bytes(w, n_tok)) {
             int rc = grow(g.part, pb, st);
@@ -623,7 +693,8 @@ static size_t part_bytes(const Fh3W *w, int n_tok, int epi) {
 }
 
 // part_ext: partial sums in caller-provided device memory (at least
-// part_bytes()), else in the library's grow-only buffer.
+// part_bytes()), else in the library's grow-only buffer.  With part_ext
+// nothing of the library's is used or allocated.
 static int product(const Fh3W *w, const void *prep, int n_tok, const float *bias, float *d_y, hipStream_t st,
                    int epi = FH3_EPI_NONE, const float *aux = nullptr, float *part_ext = nullptr) {
     if (w->type != FH3_QUANT_Q4_K || general_rows(w->in)) {
@@ -653,6 +724,13 @@ static int product(const Fh3W *w, const void *prep, int n_tok, const float *bias
         // middle M, and the GEMM with few tiles) need the partial-sum workspace
         const size_t pb = part_bytes(w, n_tok, epi);
         std::unique_lock<std::recursive_mutex> lk(g.mu, std::defer_lock);
+        if (path == FH3_HIP_PATH_GEMM && !part_ext) {
+            lk.lock();
+            bool done;
+            int rc = product_wfrag(w, prep, xs_inv, n_tok, bias, d_y, epi, aux, st, &done);
+            if (rc != FH3_OK || done) return rc;
+            lk.unlock();
+        }
         float *part = part_ext;
         if (pb && !part) {
             lk.lock();

@@ -112,6 +112,13 @@ size_t fh3k_gemm_part_bytes(int N, int K, int M, int epi);
 hipError_t fh3k_gemm_q(int type, const void *W, int64_t row_bytes, int N, int K, const void *x16,
                        const float *xs_inv, const float *bias, float *y, int M, float *part, hipStream_t st);
 int fh3k_gemm_q_takes(int type);
+// The largest Q4_K / Q5_K / Q6_K products: weights decoded into wfrag (16-byte
+// aligned, fh3k_gemm256_bytes bytes; 0 = the shape takes fh3k_gemm_epi /
+// fh3k_gemm_q), then 256 x 256 tiles.  The bits of those kernels.
+hipError_t fh3k_gemm256(int type, const void *W, int64_t row_bytes, int N, int K, const void *x16,
+                        const float *xs_inv, const float *bias, float *y, int M, int epi, const float *aux,
+                        void *wfrag, hipStream_t st);
+size_t fh3k_gemm256_bytes(int type, int N, int K, int M, int epi);
 // Prepared rows k_gemm reads for M tokens (its tiles cover 128 or 256
 // tokens; at most round_up(M, fh3k_gemm_row_pad())).
 int fh3k_gemm_rows(int M);

@@ -2334,6 +2334,382 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
 }
 
 // ---------------------------------------------------------------------------
+// k_gemm256: the largest products, from weights decoded once per call.
+//
+// k_gemm dequantises each weight once per 256 tokens and reads the
+// activations straight into registers; at thousands of tokens that work and
+// the two operands' L2 and vector-memory traffic bound it (1.1 PFLOP/s).  Here
+// k_wfrag writes the fp16 weights (k_gemm's values, bit for bit) in the
+// fragment order of X16 and the product is a plain fp16 tile product:
+//   - a 256 x 256 tile per workgroup, four wavefronts of 128 weight rows x 128
+//     tokens: 256 accumulators in AGPRs, 16 LDS reads per 64 MFMAs (half the LDS
+//     bytes per MFMA of a 128 x 64 wavefront tile, whose operands would keep
+//     the LDS port busy all the time);
+//   - v_mfma_f32_16x16x32_f16 (half the accumulator traffic of the 32x32x16 form
+//     and a higher clock under load) with the weights as A, so that a lane's four
+//     results are four neighbouring output columns;
+//   - K in stages of 32: both operands' 32 KiB go straight into LDS, four stages
+//     deep; a stage's loads are issued four stages ahead and waited for two
+//     stages ahead (1.4 us at the loaded clock: past the L2, from the
+//     Infinity Cache or HBM); fragments are read one stage ahead, so that one
+//     wavefront per SIMD never waits for LDS at a barrier.
+// The MFMAs are written as asm with the accumulator tied (the builtin's separate
+// destination made the compiler move accumulators between registers, +10 % at
+// K = 5120) and sched_barrier keeps the loads where they stand.
+// Dequantising inside this kernel instead (78 VALU per 64 MFMAs) measured 0.72
+// against 0.54 us per stage: with one wavefront per SIMD the VALU does not
+// overlap with the MFMAs.
+// K = 13824, N = 5120, 32768 tokens: 4102 us (k_gemm) -> 3262 + 30 us
+// (1.42 PFLOP/s); K = 5120, N = 15360, 8192 tokens: 1177 -> 960 + 32 us.
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr int G256_B = 256;  // tokens and weight rows of a tile
+
+// Stage ST (0..7) of a super-block is 32 k: the nibble half ST & 1 of chunk ST / 2.  Its two 16-k fragments begin at
+// fragment g256_frag of the super-block (Q6_K: see gemm_dequant).
+template <int QT, int ST>
+constexpr int g256_frag() {
+    return QT == FH3K_Q6_K ? 8 * (ST >> 2) + 2 * ((ST >> 1) & 1) + 4 * (ST & 1) : 2 * ST;
+}
+
+template <int QT, int ST>
+__device__ __forceinline__ void g256_scale(const GemmRaw<QT> &r, int h, float &D, float &C) {
+    constexpr int c = ST >> 1, nib = ST & 1;
+    if constexpr (QT == FH3K_Q6_K) {
+        const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(r.d & 0xFFFFu));
+        D = d * (float)(int)(int8_t)(uint8_t)((nib ? r.sc.y : r.sc.x) >> (8 * (2 * (c & 1) + h)));
+        C = -1056.0f * D;
+    } else {
+        q4k_group_j(r.hv, c >= 2, ((2 * c) & 3) + nib, D, C);
+    }
+}
+
+// bytes 0..7 (w = 0) or 8..15 (w = 1) of this thread's 16 quants of stage ST
+template <int QT, int ST, int w>
+__device__ __forceinline__ void g256_bytes(const GemmRaw<QT> &r, uint32_t &a, uint32_t &b) {
+    constexpr int sh = 4 * (ST & 1);
+    a = ((w ? r.qv.z : r.qv.x) >> sh) & 0x0F0F0F0Fu;
+    b = ((w ? r.qv.w : r.qv.y) >> sh) & 0x0F0F0F0Fu;
+    if constexpr (QT == FH3K_Q5_K) {
+        a |= (((w ? r.hb.z : r.hb.x) >> ST) & 0x01010101u) << 4;
+        b |= (((w ? r.hb.w : r.hb.y) >> ST) & 0x01010101u) << 4;
+    }
+    if constexpr (QT == FH3K_Q6_K) {
+        constexpr int hs = 2 * ((ST >> 1) & 1) + 4 * (ST & 1);
+        const uint32_t h0 = w ? r.hb.z : r.hb.x, h1 = w ? r.hb.w : r.hb.y;
+        a |= (hs >= 4 ? h0 >> (hs - 4) : h0 << (4 - hs)) & 0x30303030u;
+        b |= (hs >= 4 ? h1 >> (hs - 4) : h1 << (4 - hs)) & 0x30303030u;
+    }
+}
+
+
+// chunk c of the super-block at b: the pieces gemm_load_raw holds
+template <int QT>
+__device__ __forceinline__ void wfrag_load(const uint8_t *b, int c, int h, GemmRaw<QT> &r) {
+    if constexpr (QT == FH3K_Q6_K) {
+        r.qv = ld16u(b + 64 * (c >> 1) + 32 * (c & 1) + 16 * h);
+        r.hb = ld16u(b + 128 + 32 * (c >> 1) + 16 * h);
+        r.sc = *reinterpret_cast<const u32x2u *>(b + 192 + 8 * (c >> 1));
+        r.d = ld_u16(b + 208);
+    } else {
+        r.hv = ld16(b);
+        r.qv = ld16(b + (QT == FH3K_Q5_K ? 48 : 16) + 32 * c + 16 * h);
+        if constexpr (QT == FH3K_Q5_K) r.hb = ld16(b + 16 + 16 * h);
+    }
+}
+
+template <int QT, int ST>
+__device__ __forceinline__ void wfrag_stage(const GemmRaw<QT> &r, int h, half8 *out) {
+    float D, C;
+    uint32_t a, b;
+    g256_scale<QT, ST>(r, h, D, C);
+    half8 *d = out + g256_frag<QT, ST>() * 64;
+    g256_bytes<QT, ST, 0>(r, a, b);
+    d[0] = deq8_bytes(a, b, D, C);
+    g256_bytes<QT, ST, 1>(r, a, b);
+    d[32] = deq8_bytes(a, b, D, C);
+}
+
+template <int QT, int CH>
+__device__ __forceinline__ void wfrag_chunk(const GemmRaw<QT> &r, int h, half8 *out) {
+    wfrag_stage<QT, 2 * CH>(r, h, out);
+    wfrag_stage<QT, 2 * CH + 1>(r, h, out);
+}
+
+// Weights -> fp16 fragments [row block of 32][K / 16][64 slots], rows in the order
+// of k_gemm256's tiles: as they are, or (SwiGLU) groups of 64 val and their 64
+// gate rows; rows past the end repeat the last one.  A wavefront takes 32
+// rows x one super-block: 16-byte loads, 512-byte runs of stores.  Bound by
+// memory: 0.56 + 2 bytes per weight.
+template <int QT>
+__global__ __launch_bounds__(256) void k_wfrag(const uint8_t *__restrict__ W, int64_t row_bytes, int N, int K,
+                                               bool pairs, half8 *__restrict__ dst) {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int nsb = K / 256, sb = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (sb >= nsb) return;
+    int row = blockIdx.x * 32 + (lane & 31);
+    if (pairs) row = ((row >> 7) << 6) + (row & 63) + ((row & 64) ? N >> 1 : 0);
+    row = row < N ? row : N - 1;
+    constexpr int SB = QT == FH3K_Q5_K ? 176 : (QT == FH3K_Q6_K ? 210 : 144);
+    const uint8_t *b = W + (size_t)row * row_bytes + (size_t)sb * SB;
+    half8 *out = dst + ((size_t)blockIdx.x * (K / 16) + (size_t)sb * 16 + h) * 64 + (lane & 31);
+    GemmRaw<QT> r[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) wfrag_load<QT>(b, c, h, r[c]);
+    wfrag_chunk<QT, 0>(r[0], h, out);
+    wfrag_chunk<QT, 1>(r[1], h, out);
+    wfrag_chunk<QT, 2>(r[2], h, out);
+    wfrag_chunk<QT, 3>(r[3], h, out);
+}
+
+__device__ __forceinline__ void mfma4(f32x4 &c0, f32x4 &c1, f32x4 &c2, f32x4 &c3, const half8 &a, const half8 &b0,
+                                      const half8 &b1, const half8 &b2, const half8 &b3) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %4, %5, %0\n\t"
+                 "v_mfma_f32_16x16x32_f16 %1, %4, %6, %1\n\t"
+                 "v_mfma_f32_16x16x32_f16 %2, %4, %7, %2\n\t"
+                 "v_mfma_f32_16x16x32_f16 %3, %4, %8, %3"
+                 : "+a"(c0), "+a"(c1), "+a"(c2), "+a"(c3)
+                 : "v"(a), "v"(b0), "v"(b1), "v"(b2), "v"(b3));
+}
+
+// DMA of a stage (32 k: fragments f, f + 1 of 8 + 8 blocks of 32 rows): 32 KiB, 8 loads per wavefront
+__device__ __forceinline__ void g256_dma(__amdgpu_buffer_rsrc_t r, int lane16, int tbs, int f, int blk, int u,
+                                         half8 (*dst)[64]) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)&dst[blk * 2 + u][0], 16, lane16,
+                                             blk * tbs + (f + u) * 1024, 0, 0);
+}
+
+// One stage: its 64 MFMAs; the next stage's fragments read from wl, xl; the
+// DMA of the stage with fragments fd, fd + 1 into dst.
+__device__ __forceinline__ void g256_stage(const half8 (&wf)[8], const half8 (&xf)[8], half8 (&wn)[8], half8 (&xn)[8],
+                                           const half8 *wl, const half8 *xl, f32x4 (&acc)[8][8],
+                                           __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t wr, int lane16, int tbs,
+                                           int fd, int wave, half8 (*dst)[64]) {
+#pragma unroll
+    for (int g = 0; g < 16; g++) {
+        const int i = g >> 1, j = 4 * (g & 1);
+        mfma4(acc[i][j], acc[i][j + 1], acc[i][j + 2], acc[i][j + 3], wf[i], xf[j], xf[j + 1], xf[j + 2], xf[j + 3]);
+        if (g < 4) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int n = 2 * g + u;
+                xn[n] = xl[(n >> 1) * 128 + 16 * (n & 1)];
+            }
+        } else if (g < 12) {
+            const int n = g - 4;
+            wn[n] = wl[(n >> 1) * 128 + 16 * (n & 1)];
+        }
+        if ((g & 1) == 0) {
+            const int u = g >> 1;  // 0..7: X blocks 2 wave, 2 wave + 1, then W
+            if (u < 4) g256_dma(xr, lane16, tbs, fd, 2 * wave + (u >> 1), u & 1, dst + 16);
+            else g256_dma(wr, lane16, tbs, fd, 2 * wave + ((u >> 1) & 1), u & 1, dst);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(0x4070);  // vmcnt(16) lgkmcnt(0): all but the last two stages' loads have landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Epilogue of 64 tokens x 128 weight rows staged in a wavefront's 32 KiB of LDS,
+// [64 tokens][32 chunks of 4 rows] with chunk c of token t at c ^ (t & 15) (no
+// bank conflicts, written or read): 16-byte stores of whole rows where the output
+// allows them, else one float per lane, neighbouring lanes on neighbouring
+// columns.  Rolled loops: unrolled over the accumulators the code ran once per tile
+// and its instruction fetches took longer than the stores (17 us a tile, now 7).
+template <int EPI>
+__device__ __forceinline__ void g256_rows(const f32x4 *stg, int lane, int tw, int ob, int N,
+                                          const float *__restrict__ xs_inv, const float *__restrict__ bias,
+                                          float *__restrict__ Y, int M, const float *__restrict__ aux) {
+    constexpr bool SW = EPI == EPI_SWIGLU;
+    constexpr int COLS = SW ? 64 : 128;      // output columns
+    constexpr int TPI = 256 / COLS, UN = 4;  // tokens per pass of 16-byte pieces, passes per iteration
+    const int F = N >> 1, width = SW ? F : N;
+    const float xsl = tw + lane < M ? xs_inv[tw + lane] : 0.f;
+    if ((width & 3) == 0 && ((reinterpret_cast<uintptr_t>(Y) | reinterpret_cast<uintptr_t>(aux)) & 15) == 0) {
+        const int ch = lane & (COLS / 4 - 1), tq = lane / (COLS / 4);
+        const int o = ob + 4 * ch;
+        const bool oin = o < width;  // the four columns are inside together
+        f32x4 bv = {0.f, 0.f, 0.f, 0.f}, bg = bv;
+        if (bias && oin) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                bv[v] = bias[o + v];
+                if (SW) bg[v] = bias[F + o + v];
+            }
+        }
+#pragma unroll 1
+        for (int it = 0; it < 64; it += TPI * UN) {
+            f32x4 y[UN];
+#pragma unroll
+            for (int u = 0; u < UN; u++) {
+                const int tl = it + u * TPI + tq;
+                const float xs = __shfl(xsl, tl);
+                const f32x4 a = stg[tl * 32 + (ch ^ (tl & 15))];
+                f32x4 g = a;
+                if (SW) g = stg[tl * 32 + ((16 + ch) ^ (tl & 15))];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    y[u][v] = a[v] * xs + bv[v];
+                    if (SW) y[u][v] = y[u][v] * silu_f32(g[v] * xs + bg[v]);
+                }
+            }
+            const size_t at = (size_t)(tw + it + tq) * width + o, step = (size_t)TPI * width;
+            bool in[UN];
+#pragma unroll
+            for (int u = 0; u < UN; u++) in[u] = oin && tw + it + tq + u * TPI < M;
+            if constexpr (EPI == EPI_GATE_RES) {
+                f32x4 g[UN] = {}, c[UN] = {};
+#pragma unroll
+                for (int u = 0; u < UN; u++)
+                    if (in[u]) {
+                        g[u] = *reinterpret_cast<const f32x4 *>(aux + at + u * step);
+                        c[u] = *reinterpret_cast<const f32x4 *>(Y + at + u * step);
+                    }
+#pragma unroll
+                for (int u = 0; u < UN; u++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) y[u][v] = __builtin_fmaf(g[u][v], y[u][v], c[u][v]);
+            }
+#pragma unroll
+            for (int u = 0; u < UN; u++)
+                if (in[u]) *reinterpret_cast<f32x4 *>(Y + at + u * step) = y[u];
+        }
+        return;
+    }
+    const float *sf = reinterpret_cast<const float *>(stg);
+#pragma unroll 1
+    for (int k = 0; k < COLS / 64; k++) {
+        const int col = 64 * k + lane, o = ob + col, ch = col >> 2, e = col & 3;
+        const bool oin = o < width;
+        const float bv = bias && oin ? bias[o] : 0.f, bg = SW && bias && oin ? bias[F + o] : 0.f;
+#pragma unroll 1
+        for (int it = 0; it < 64; it += 8) {
+            float y[8], g[8] = {}, c[8] = {};
+            const size_t at = (size_t)(tw + it) * width + o;
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int tl = it + u;
+                const float xs = __shfl(xsl, tl);
+                y[u] = sf[(tl * 32 + (ch ^ (tl & 15))) * 4 + e] * xs + bv;
+                if (SW) y[u] = y[u] * silu_f32(sf[(tl * 32 + ((16 + ch) ^ (tl & 15))) * 4 + e] * xs + bg);
+                if (EPI == EPI_GATE_RES && oin && tw + tl < M) {
+                    g[u] = aux[at + (size_t)u * width];
+                    c[u] = Y[at + (size_t)u * width];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (oin && tw + it + u < M)
+                    Y[at + (size_t)u * width] = EPI == EPI_GATE_RES ? __builtin_fmaf(g[u], y[u], c[u]) : y[u];
+        }
+    }
+}
+
+// Wait states between MFMAs and other instructions that touch the
+// accumulators, which the compiler does not see behind the asm.
+#define G256_ACC_ROW(i)                                                                                        \
+    "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]),      \
+        "+a"(acc[i][6]), "+a"(acc[i][7])
+__device__ __forceinline__ void g256_settle(f32x4 (&acc)[8][8]) {
+#pragma unroll
+    for (int i = 0; i < 7; i++) asm volatile("" : G256_ACC_ROW(i));
+    asm volatile("s_nop 15\n\ts_nop 15" : G256_ACC_ROW(7));
+#pragma unroll
+    for (int i = 0; i < 7; i++) asm volatile("" : G256_ACC_ROW(i));
+}
+#undef G256_ACC_ROW
+
+// Q6: the stages of a K step of 128 in k_gemm's order for Q6_K (fragments 0, 4, 2,
+// 6 of each eight: see gemm_dequant), so that the sums round alike.
+template <bool Q6>
+__global__ __launch_bounds__(256, 1) void k_gemm256(const half8 *__restrict__ W16, int N, int K,
+                                                    const half8 *__restrict__ X16, const float *__restrict__ xs_inv,
+                                                    const float *__restrict__ bias, float *__restrict__ Y, int M,
+                                                    int m_tiles, int n_tiles, int epi,
+                                                    const float *__restrict__ aux) {
+    __shared__ half8 l0[32][64], l1[32][64], l2[32][64], l3[32][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave & 1, wm = wave >> 1;
+    const int total = m_tiles * n_tiles, id = blockIdx.x, per = total >> 3;
+    const int L = (id < per * 8) ? (id & 7) * per + (id >> 3) : id;
+    // Bands of four token tiles, column by column, so that the 32 tiles an XCD
+    // runs at a time are 4 x 8: 12 operand tiles through its L2 per K step where a
+    // token-major order needs 33 (8192 x 5120 -> 15360: 1094 -> 990 us; bands of 2
+    // or 8: 1015 / 990).
+    constexpr int GB = 4;
+    const int band = L / (GB * n_tiles), gs = min(GB, m_tiles - band * GB), in = L - band * GB * n_tiles;
+    const int nt = in / gs, mt = band * GB + in - nt * gs;
+    const int m0 = mt * G256_B, n0 = nt * G256_B;
+
+    const int tbs = (K / 16) * 1024;
+    const __amdgpu_buffer_rsrc_t xr = buf_rsrc(X16 + (size_t)(m0 / 32) * (K / 16) * 64, 8u * (uint32_t)tbs);
+    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W16 + (size_t)(n0 / 32) * (K / 16) * 64, 8u * (uint32_t)tbs);
+    const int lane16 = lane * 16;
+    constexpr int f1 = Q6 ? 4 : 2, f2 = Q6 ? 2 : 4;
+    const int fs = frag32_slot(lane);
+    const int wo = wn * 8 * 64 + fs, xo = (16 + wm * 8) * 64 + fs;
+
+    f32x4 acc[8][8];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    half8 fw0[8], fx0[8], fw1[8], fx1[8];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        half8(*d)[64] = s == 0 ? l0 : (s == 1 ? l1 : (s == 2 ? l2 : l3));
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int f = s == 1 ? f1 : (s == 2 ? f2 : 2 * s);
+            g256_dma(xr, lane16, tbs, f, 2 * wave + (u >> 1), u & 1, d + 16);
+            g256_dma(wr, lane16, tbs, f, 2 * wave + (u >> 1), u & 1, d);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x4070);  // stages 0 and 1
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < 8; n++) {
+        fw0[n] = (&l0[0][0])[wo + (n >> 1) * 128 + 16 * (n & 1)];
+        fx0[n] = (&l0[0][0])[xo + (n >> 1) * 128 + 16 * (n & 1)];
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();        // every wavefront holds stage 0: its buffer is free
+    __builtin_amdgcn_sched_barrier(0);
+    g256_settle(acc);
+    const int S = K / 32;
+    for (int s = 0; s < S; s += 4) {
+        const int d = 2 * (s + 4 < S ? s + 4 : s);
+        g256_stage(fw0, fx0, fw1, fx1, &l1[0][0] + wo, &l1[0][0] + xo, acc, xr, wr, lane16, tbs, d, wave, l0);
+        g256_stage(fw1, fx1, fw0, fx0, &l2[0][0] + wo, &l2[0][0] + xo, acc, xr, wr, lane16, tbs, d + f1, wave, l1);
+        g256_stage(fw0, fx0, fw1, fx1, &l3[0][0] + wo, &l3[0][0] + xo, acc, xr, wr, lane16, tbs, d + f2, wave, l2);
+        g256_stage(fw1, fx1, fw0, fx0, &l0[0][0] + wo, &l0[0][0] + xo, acc, xr, wr, lane16, tbs, d + 6, wave, l3);
+    }
+    g256_settle(acc);
+    __builtin_amdgcn_s_waitcnt(0x0070);  // every load into LDS has landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 *stg = reinterpret_cast<f32x4 *>(wave == 0 ? l0 : (wave == 1 ? l1 : (wave == 2 ? l2 : l3)));
+    const bool sw = epi == EPI_SWIGLU;
+    const int tw = m0 + 128 * wm, ob = sw ? nt * 128 + 64 * wn : n0 + 128 * wn;
+    const int l16 = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) stg[(16 * j + l16) * 32 + ((4 * i + q) ^ l16)] = acc[i][4 * hf + j];
+        __builtin_amdgcn_wave_barrier();
+        if (sw) g256_rows<EPI_SWIGLU>(stg, lane, tw + 64 * hf, ob, N, xs_inv, bias, Y, M, aux);
+        else if (epi == EPI_GATE_RES) g256_rows<EPI_GATE_RES>(stg, lane, tw + 64 * hf, ob, N, xs_inv, bias, Y, M, aux);
+        else g256_rows<EPI_NONE>(stg, lane, tw + 64 * hf, ob, N, xs_inv, bias, Y, M, aux);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Weights of the other types (the reference's fh3_matmul takes every type its
 // fh3_dequant decodes, src/core/fh3_ops.c:325-333).  They are decoded once per
 // call to fp16 rows W16[N][K] -- the reference's fp32 value rounded once to
@@ -3439,6 +3815,64 @@ extern "C" hipError_t fh3k_gemm_q(int type, const void *W, int64_t row_bytes, in
     if (type == FH3K_Q6_K)
         return launch_gemm<FH3K_Q6_K>(W, row_bytes, N, K, x16, xs_inv, bias, y, M, EPI_NONE, nullptr, part, st);
     return hipErrorInvalidValue;
+}
+
+template <int QT>
+static hipError_t launch_gemm256(const void *W, int64_t row_bytes, int N, int K, const void *x16, const float *xs_inv,
+                                 const float *bias, float *y, int M, int epi, const float *aux, void *wfrag,
+                                 hipStream_t st) {
+    const int m_tiles = (M + G256_B - 1) / G256_B;
+    const int n_tiles = epi == EPI_SWIGLU ? (N / 2 + 127) / 128 : (N + G256_B - 1) / G256_B;
+    hipLaunchKernelGGL(k_wfrag<QT>, dim3((unsigned)(n_tiles * 8), (unsigned)((K / 256 + 3) / 4)), dim3(256), 0, st,
+                       (const uint8_t *)W, row_bytes, N, K, epi == EPI_SWIGLU, (half8 *)wfrag);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_gemm256<QT == FH3K_Q6_K>, dim3((unsigned)(m_tiles * n_tiles)), dim3(256), 0, st, (const half8 *)wfrag, N, K,
+                       (const half8 *)x16, xs_inv, bias, y, M, m_tiles, n_tiles, epi, aux);
+    return hipGetLastError();
+}
+
+// Estimated times of both forms in us at K = 5120 (they scale with K), from
+// rounds of the 256 CUs.  k_gemm: 157 us per full round of 512 tiles of 256 x
+// 128, 64 + 0.18 us per tile of the last one; k_gemm256: 119 us per full round
+// of 256, 105 for the last, and the decode, 2.56 bytes per weight at 5 TB/s.
+// Measured, k_gemm against both launches, us: K = 5120, N = 17408 at 1024 /
+// 1500 / 2048 / 3016 tokens 233 / 285 / 382 / 536 against 242 / 254 / 380 / 495;
+// N = 5120 at 2048 / 4096 / 8192 tokens 128 / 236 / 406 against 114 / 219 /
+// 343; N = 1024 / 2048 at 4096 tokens 86 / 101 against 93 / 105; 6000 tokens,
+// 1024 -> 2000 48 against 36.  Only where k_gemm does not split K: the two then
+// give the same bits, which one a call takes cannot be told from its result.
+static bool gemm256_wins(int N, int K, int M, int epi) {
+    int C, S;
+    gemm_split(M, N, K, epi, C, S);
+    if (M < 1024 || S > 1) return false;
+    const int64_t mt = (M + 255) / 256;
+    const int64_t t0 = mt * (epi == EPI_SWIGLU ? (N / 2) / 64 : (N + GEMM_BN - 1) / GEMM_BN);
+    const int64_t t1 = mt * (epi == EPI_SWIGLU ? (N / 2 + 127) / 128 : (N + G256_B - 1) / G256_B);
+    const double one = t0 / 512 * 157.0 + (t0 % 512 ? 64.0 + 0.18 * (double)(t0 % 512) : 0.0);
+    const double two = t1 / 256 * 119.0 + (t1 % 256 ? 105.0 : 0.0) + (double)N * 5120.0 * 2.56 / 5.0e6;
+    return two < 0.98 * one;
+}
+
+constexpr size_t G256_MAX_BYTES = (size_t)1 << 30;  // fp16 fragments a product may ask for
+
+extern "C" size_t fh3k_gemm256_bytes(int type, int N, int K, int M, int epi) {
+    if (type != FH3K_Q4_K && type != FH3K_Q5_K && type != FH3K_Q6_K) return 0;
+    if (K < 256 || K % 256 || N < 1 || (epi == EPI_SWIGLU && N % 128) || !gemm256_wins(N, K, M, epi)) return 0;
+    const int n_tiles = epi == EPI_SWIGLU ? (N / 2 + 127) / 128 : (N + G256_B - 1) / G256_B;
+    const size_t bytes = (size_t)n_tiles * G256_B * (size_t)K * 2;
+    return bytes <= G256_MAX_BYTES ? bytes : 0;
+}
+
+extern "C" hipError_t fh3k_gemm256(int type, const void *W, int64_t row_bytes, int N, int K, const void *x16,
+                                   const float *xs_inv, const float *bias, float *y, int M, int epi, const float *aux,
+                                   void *wfrag, hipStream_t st) {
+    if (!wfrag || fh3k_gemm256_bytes(type, N, K, M, epi) == 0) return hipErrorInvalidValue;
+    if (type == FH3K_Q4_K)
+        return launch_gemm256<FH3K_Q4_K>(W, row_bytes, N, K, x16, xs_inv, bias, y, M, epi, aux, wfrag, st);
+    if (type == FH3K_Q5_K)
+        return launch_gemm256<FH3K_Q5_K>(W, row_bytes, N, K, x16, xs_inv, bias, y, M, epi, aux, wfrag, st);
+    return launch_gemm256<FH3K_Q6_K>(W, row_bytes, N, K, x16, xs_inv, bias, y, M, epi, aux, wfrag, st);
 }
 
 // ---------------------------------------------------------------------------

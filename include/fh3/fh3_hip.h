@@ -226,7 +226,12 @@ int fh3_hip_graph_destroy(void *graph_exec);
  * activations of fh3_hip_matmul_dev / fh3_hip_matmul_epi_dev (prepared = 0)
  * plus the partial sums of the split-K kernels; with prepared = 1 the same for
  * fh3_hip_matmul_prepared_dev / _prepared_epi_dev.  epi as below.  Under the
- * current fh3_hip_set_path setting. */
+ * current fh3_hip_set_path setting.  Not counted: the fp16 weights (out * in *
+ * 2 bytes, at most 1 GiB) that a Q4_K, Q5_K or Q6_K product of about 1024
+ * tokens or more decodes when it can.  One buffer, kept until
+ * fh3_hip_shutdown, serves all streams (their products wait for one another on
+ * the device); under capture, and where the memory is not to be had, the
+ * weights are read in place instead, with the same results. */
 size_t fh3_hip_matmul_workspace_bytes(const Fh3W *w, int n_tok, int epi, int prepared);
 
 /* The no-allocation product, for callers that cannot allocate device memory
