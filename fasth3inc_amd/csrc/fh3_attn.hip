@@ -29,6 +29,7 @@ namespace {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
 constexpr int ATT_KT = 64;   // keys per tile
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
     __shared__ _Float16 sk[2][ATT_KT][KROW];
     __shared__ _Float16 sv[2][HD][VROW];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hf = lane >> 5;
 
     // XCD-aware order: consecutive workgroup ids land on different XCDs, so
@@ -275,6 +276,10 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
         const half8 *qp = (const half8 *)(Qp + ((size_t)h * n_pad + q0 + l32) * HD + 8 * hf);
 #pragma unroll
         for (int kk = 0; kk < KS; kk++) qf[kk] = qp[2 * kk];
+        // Wait for them here: left to the loop, their waits stand among each
+        // tile's products and drain the next tile's loads as well.
+#pragma unroll
+        for (int kk = 0; kk < KS; kk++) asm volatile("" : "+v"(qf[kk]));
     }
 
     // key tiles to visit: 0 .. nkt-1 (dense) or the block's list (sparse)
@@ -284,7 +289,27 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
         lst = sp.lists + (size_t)L * sp.T;
         nkt = sp.list_len[L];
     }
-    auto tile_of = [&](int e) { return SPARSE ? (int)(lst[e] & 0x3FFF) : e; };
+    // Sparse: 64 list entries at a time and their tiles' token counts, one per
+    // lane, read from there as scalars (loaded when used, an entry and a count
+    // cost each tile two memory latencies, and their waits drained the tile loads)
+    uint32_t ents = 0;
+    int cnts = 0;
+    auto load_entries = [&](int e) {
+        const int i = e + lane < nkt ? e + lane : nkt - 1;
+        ents = lst[i];
+        cnts = sp.cnt[ents & 0x3FFF];
+    };
+    // entry e: a sparse list's entry or the key tile, and its number of keys
+    auto entry = [&](int e, int &ent, int &keys) {
+        if (SPARSE) {
+            if ((e & 63) == 0) load_entries(e);
+            ent = __builtin_amdgcn_readlane((int)ents, e & 63);
+            keys = __builtin_amdgcn_readlane(cnts, e & 63);
+        } else {
+            ent = e;
+            keys = n - e * ATT_KT;
+        }
+    };
 
     half8 rk[KCH], rv[KCH];
     auto load_tile = [&](int j) {
@@ -311,28 +336,34 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
     f32x16 o[DB];
 #pragma unroll
     for (int i = 0; i < DB; i++) o[i] = f32x16{};
-    float m = -INFINITY, lsum = 0.f;
+    f32x16 nm = {};     // minus the query's softmax offset, as an accumulator to start from
+    float lsum = 0.f;
+    float thr = -INFINITY;  // before the first tile: its maximum becomes the offset, whatever it is
 
+    int ent = 0, kv = 0;  // kv: keys in the tile (>= 1)
     if (nkt > 0) {
-        load_tile(tile_of(0));
+        entry(0, ent, kv);
+        load_tile(SPARSE ? ent & 0x3FFF : ent);
         store_tile(0);
     }
     __syncthreads();
     for (int e = 0; e < nkt; e++) {
         const int b = e & 1;
-        const int j = tile_of(e);
-        if (e + 1 < nkt) load_tile(tile_of(e + 1));
-        // valid keys in this tile (>= 1); in sparse mode, whether this pair of
-        // wavefronts' query tile selected it (wave-uniform)
-        const int kv = SPARSE ? sp.cnt[j] : n - j * ATT_KT;
-        const bool active = SPARSE ? ((lst[e] >> (14 + (wave >> 1))) & 1) != 0 : true;
+        int ent_n = 0, kv_n = 0;
+        if (e + 1 < nkt) {
+            entry(e + 1, ent_n, kv_n);
+            load_tile(SPARSE ? ent_n & 0x3FFF : ent_n);
+        }
+        // sparse: whether this pair of wavefronts' query tile selected it (wave-uniform)
+        const bool active = SPARSE ? ((ent >> (14 + (wave >> 1))) & 1) != 0 : true;
         if (active) {
             // dense: raised wave priority through the tile's matrix and softmax
             // work (the other wavefront on the SIMD is then mostly loading or
             // waiting; +1-2 %; the sparse walk loses with it)
             if constexpr (!SPARSE) __builtin_amdgcn_s_setprio(2);
-            // S^T[key][query] for the 64 keys: two 32-key accumulators
-            f32x16 s[2] = {f32x16{}, f32x16{}};
+            // S^T[key][query] - m for the 64 keys: two 32-key accumulators that
+            // start at -m, so that the softmax needs no subtraction
+            f32x16 s[2] = {nm, nm};
 #pragma unroll
             for (int kk = 0; kk < KS; kk++) {
 #pragma unroll
@@ -343,49 +374,57 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
             }
             // lane holds keys 32 st + 8 (v/4) + 4 hf + v%4 of query q0 + l32
             if (kv < ATT_KT) {
+                const int kh = kv - 4 * hf;
 #pragma unroll
                 for (int st = 0; st < 2; st++)
 #pragma unroll
-                    for (int v = 0; v < 16; v++)
-                        if (32 * st + 8 * (v >> 2) + 4 * hf + (v & 3) >= kv) s[st][v] = -INFINITY;
+                    for (int v = 0; v < 16; v++) s[st][v] = kh > 32 * st + 8 * (v >> 2) + (v & 3) ? s[st][v] : -INFINITY;
             }
             float mt = s[0][0];
 #pragma unroll
             for (int v = 1; v < 16; v++) mt = fmaxf(mt, s[0][v]);
 #pragma unroll
             for (int v = 0; v < 16; v++) mt = fmaxf(mt, s[1][v]);
-            mt = wave_swap_max(mt);
-            const bool grow = mt > m + ATT_TAU;
-            if (__ballot(grow)) {  // wave-uniform: some query's offset must rise
-                const float mn = grow ? mt : m;
-                const float alpha = __builtin_amdgcn_exp2f(m - mn);
-                m = mn;
+            // Only where some lane's own maximum asks for it do the two halves
+            // of a query compare theirs (wave-uniform).
+            if (__ballot(mt > thr)) {
+                mt = wave_swap_max(mt);
+                const float up = mt > thr ? mt : 0.f;
+                const float alpha = thr < 0.f ? 0.f : __builtin_amdgcn_exp2f(-up);
+#pragma unroll
+                for (int v = 0; v < 16; v++) nm[v] -= up;
+                thr = ATT_TAU;
                 lsum *= alpha;
 #pragma unroll
                 for (int i = 0; i < DB; i++) o[i] *= alpha;
+#pragma unroll
+                for (int st = 0; st < 2; st++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) s[st][v] -= up;
             }
 #pragma unroll
             for (int st = 0; st < 2; st++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) s[st][v] = __builtin_amdgcn_exp2f(s[st][v] - m);
+                for (int v = 0; v < 16; v++) s[st][v] = __builtin_amdgcn_exp2f(s[st][v]);
 
             // P^T fragments: 16-key step t = values 4g..4g+7 of accumulator
             // t/2, g = 2 (t % 2); they pair with V^T stored in the vt_key
             // order.  The row sum is taken over the same fp16 values the
             // product uses.
             half8 pf[4];
-#pragma unroll
-            for (int tt = 0; tt < 4; tt++) {
-#pragma unroll
-                for (int q = 0; q < 8; q++) pf[tt][q] = (_Float16)s[tt >> 1][8 * (tt & 1) + q];
-            }
             float ps[2] = {0.f, 0.f};
 #pragma unroll
-            for (int tt = 0; tt < 4; tt++)
+            for (int tt = 0; tt < 4; tt++) {
+                uint32_t w[4];
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    ps[q & 1] = __builtin_amdgcn_fdot2(half2v{pf[tt][2 * q], pf[tt][2 * q + 1]}, half2v{1, 1},
-                                                       ps[q & 1], false);
+                for (int q = 0; q < 4; q++) {
+                    w[q] = __builtin_bit_cast(uint32_t, half2v{(_Float16)s[tt >> 1][8 * (tt & 1) + 2 * q],
+                                                               (_Float16)s[tt >> 1][8 * (tt & 1) + 2 * q + 1]});
+                    asm("" : "+v"(w[q]));  // one pair, not converted once for each use
+                    ps[q & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, w[q]), half2v{1, 1}, ps[q & 1], false);
+                }
+                pf[tt] = __builtin_bit_cast(half8, u32x4{w[0], w[1], w[2], w[3]});
+            }
             lsum += ps[0] + ps[1];
 #pragma unroll
             for (int db = 0; db < DB; db++) {
@@ -398,6 +437,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
         }
         if constexpr (!SPARSE) __builtin_amdgcn_s_setprio(0);
         if (e + 1 < nkt) store_tile(b ^ 1);
+        ent = ent_n;
+        kv = kv_n;
         __syncthreads();
     }
 
