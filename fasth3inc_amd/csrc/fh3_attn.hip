@@ -50,11 +50,8 @@ constexpr float ATT_TAU = 8.0f;
 // Order of the keys inside each 16-key block of Vt.  The P^T operand of the
 // PV product is taken straight from the S^T accumulator, where lane half hf
 // holds keys {4hf..4hf+3, 8+4hf..8+4hf+3} of each 16-key block; storing V^T
-// in that order lets one 16-byte LDS read feed the matching A operand.
-__device__ __forceinline__ int vt_key(int p) {
-    const int b = p & 15;
-    return (p & ~15) + ((b & 3) | ((b & 4) << 1) | ((b & 8) >> 1));
-}
+// in that order lets one 16-byte LDS read feed the matching A operand:
+// position b of a block holds key (b & 3) | (b & 4) << 1 | (b & 8) >> 1.
 
 // Tile pooling (video sparse attention): with a gather map each prep
 // workgroup holds exactly one 64-slot tile, so it also writes the tile's
@@ -69,152 +66,246 @@ struct Pool {
     int T;
 };
 
-// sum over the first cnt rows of sx, in row order, times w (thread d < HD)
+// LDS row of the 64 staged rows: eight segments of HD/8 floats, one per thread
+// of a row, each padded by four and the row padded again, so that the eight
+// lanes of a 16-byte access (a row's segments, or eight neighbours) and the 16
+// columns x 4 rows of V's transposed reads spread over the banks.
+template <int HD> constexpr int prep_pitch() { return HD + 8 * 4 + 4; }
+template <int HD> __device__ __forceinline__ int prep_at(int r, int d) {
+    constexpr int DPT = HD / 8;
+    return r * prep_pitch<HD>() + (d / DPT) * (DPT + 4) + d % DPT;
+}
+
+// sum over the first cnt rows of sx, in row order, times w (thread d < HD):
+// sixteen rows' reads at a time ahead of the chain of additions
 template <int HD>
-__device__ __forceinline__ void pool_rows(const float (*sx)[HD + 4], int cnt, float w, float *dst) {
+__device__ __forceinline__ void pool_rows(const float *sx, int cnt, float w, float *dst) {
     const int d = threadIdx.x;
     if (d < HD) {
         float a = 0.f;
-        for (int r = 0; r < cnt; r++) a = a + sx[r][d] * w;
+        int r = 0;
+        for (; r + 16 <= cnt; r += 16) {
+            float b[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) b[i] = sx[prep_at<HD>(r + i, d)];
+#pragma unroll
+            for (int i = 0; i < 16; i++) a = a + b[i] * w;
+        }
+        for (; r < cnt; r++) a = a + sx[prep_at<HD>(r, d)] * w;
         dst[d] = a;
     }
 }
 
-template <int HD>
-__global__ __launch_bounds__(256) void k_attn_prep(const float *__restrict__ q, const float *__restrict__ k,
+// Lane c of each eight holds chunks 2c and 2c + 1 (half8 o[0], o[1]) of its
+// row's 16; afterwards o[0] of the eight lanes are chunks 0..7 and o[1] chunks
+// 8..15, so that each store covers 128 consecutive bytes: lane c and lane 7 - c
+// exchange one.  at: which chunks the lane then holds.
+__device__ __forceinline__ void pair_chunks(half8 (&o)[2], int c, int (&at)[2]) {
+    const bool up = c >= 4;
+    u32x4 a = __builtin_bit_cast(u32x4, o[0]), b = __builtin_bit_cast(u32x4, o[1]);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t send = up ? a[e] : b[e];
+        const uint32_t got = (uint32_t)__builtin_amdgcn_mov_dpp((int)send, 0x141, 0xF, 0xF, true);  // row_half_mirror
+        a[e] = up ? got : a[e];
+        b[e] = up ? b[e] : got;
+    }
+    o[0] = __builtin_bit_cast(half8, a), o[1] = __builtin_bit_cast(half8, b);
+    at[0] = up ? 15 - 2 * c : 2 * c, at[1] = up ? 2 * c + 1 : 14 - 2 * c;
+}
+
+// The work is bound by memory: 12 bytes read and 6 written per element, and the
+// rope tables, which for one head are larger than q.  One workgroup takes a tile of
+// 64 slots of G consecutive heads: rows are loaded 16 bytes per lane in order, one
+// operand ahead of the one in work, and reach the threads (eight to a row,
+// HD/8 channels each) through LDS; each thread keeps its channels' table values
+// for all q and k of its heads; a rope partner is normalised again from the raw
+// row, which takes the place of another pass through LDS.  n = 16384 x 40 heads:
+// 570 -> 292 us (5.2 TB/s); with tile pooling, n = 12922 x 56 heads: 746 -> 361 us
+// (before: 128-byte runs per lane, one operand at a time, tables for each head).
+// ANYROT: rope with rot % 8 != 0, channel by channel with the tables read in place.
+template <int HD, bool ANYROT>
+__global__ __launch_bounds__(512, 4) void k_attn_prep(const float *__restrict__ q, const float *__restrict__ k,
                                                    const float *__restrict__ v, int64_t ld, int64_t ldv, int n,
-                                                   const int *__restrict__ gather,
+                                                   int heads, int G, const int *__restrict__ gather,
                                                    const float *__restrict__ qn_w, const float *__restrict__ kn_w,
                                                    float eps, const float *__restrict__ cosb,
                                                    const float *__restrict__ sinb, int rot, float qscale,
                                                    int n_pad, _Float16 *__restrict__ Qp, _Float16 *__restrict__ Kp,
                                                    _Float16 *__restrict__ Vt, Pool pl) {
-    constexpr int DPT = HD / 4;
-    __shared__ float sx[ATT_PREP_T][HD + 4];
-    const int t = threadIdx.x, r = t >> 2, c = t & 3;
-    const int slot = blockIdx.x * ATT_PREP_T + r, h = blockIdx.y;
-    const int tok = gather ? gather[slot] : (slot < n ? slot : -1);
-    const int d0 = c * DPT;
-
-    for (int which = 0; which < 2; which++) {
-        const float *src = which ? k : q;
-        const float *nw = which ? kn_w : qn_w;
-        float x[DPT];
-        if (tok >= 0) {
-            const f32x4 *p = (const f32x4 *)(src + (size_t)tok * ld + (size_t)h * HD + d0);
+    constexpr int DPT = HD / 8, C4 = DPT / 4;
+    constexpr int LPR = HD / 4, RPP = 512 / LPR, PASS = ATT_PREP_T / RPP;  // lanes per row, rows per pass, passes
+    __shared__ __align__(16) float sx[ATT_PREP_T * prep_pitch<HD>()];
+    __shared__ __align__(16) float snw[2][HD];
+    const int t = threadIdx.x, c = t & 7, d0 = c * DPT;
+    const int tile = blockIdx.x;
+    const int h0 = blockIdx.y * G, hn = heads - h0 < G ? heads - h0 : G;
+    auto token = [&](int sl) { return gather ? gather[sl] : (sl < n ? sl : -1); };
+    const int tok = token(tile * ATT_PREP_T + (t >> 3));
+    const int lr = t / LPR, ld0 = (t % LPR) * 4;  // the row and channels this thread loads
+    int ltok[PASS];
 #pragma unroll
-            for (int i = 0; i < DPT / 4; i++) {
-                const f32x4 u = p[i];
+    for (int i = 0; i < PASS; i++) ltok[i] = token(tile * ATT_PREP_T + lr + RPP * i);
+
+    f32x4 nx[PASS];  // the next operand's rows
+    auto load = [&](int which, int h) {
+        const float *src = (which == 2 ? v : which ? k : q) + (size_t)h * HD + ld0;
+        const int64_t l = which == 2 ? ldv : ld;
+#pragma unroll
+        for (int i = 0; i < PASS; i++) {
+            int tk = ltok[i];
+            asm volatile("" : "+v"(tk));  // addresses made here, not kept for each operand through the loops
+            nx[i] = tk >= 0 ? *(const f32x4 *)(src + tk * l) : f32x4{};
+        }
+    };
+    load(0, h0);
+    if (t < HD) {
+        snw[0][t] = qn_w ? qn_w[t] : 1.f;
+        snw[1][t] = kn_w ? kn_w[t] : 1.f;
+    }
+    const bool rope4 = !ANYROT && cosb;  // rot % 8 == 0: 4-channel chunks never straddle half or rot
+    f32x4 ct[C4], st[C4];
+#pragma unroll
+    for (int i = 0; i < C4; i++) {
+        ct[i] = st[i] = f32x4{};
+        if (rope4 && tok >= 0 && d0 + 4 * i < rot) {
+            ct[i] = *(const f32x4 *)(cosb + (size_t)tok * rot + d0 + 4 * i);
+            st[i] = *(const f32x4 *)(sinb + (size_t)tok * rot + d0 + 4 * i);
+        }
+    }
+
+    for (int hi = 0; hi < hn; hi++) {
+        const int h = h0 + hi;
+#pragma unroll 1
+        for (int which = 0; which < 3; which++) {
+            __syncthreads();  // the last operand's readers are done
+#pragma unroll
+            for (int i = 0; i < PASS; i++) *(f32x4 *)&sx[prep_at<HD>(lr + RPP * i, ld0)] = nx[i];
+            if (which < 2)
+                load(which + 1, h);
+            else if (hi + 1 < hn)
+                load(0, h + 1);
+            __syncthreads();
+            if (which == 2) break;
+            int r = t >> 3, half = rot >> 1;
+            asm volatile("" : "+v"(r), "+s"(half));  // as in load()
+            const bool norm = (which ? kn_w : qn_w) != nullptr;
+            const float *nw = snw[which];
+            float x[DPT];
+#pragma unroll
+            for (int i = 0; i < C4; i++) {
+                const f32x4 u = *(const f32x4 *)&sx[prep_at<HD>(r, d0) + 4 * i];
                 x[4 * i] = u[0], x[4 * i + 1] = u[1], x[4 * i + 2] = u[2], x[4 * i + 3] = u[3];
             }
-        } else {
+            float inv = 1.f;
+            if (norm) {
+                // four chains of HD/4 channels: the odd thread of a pair goes on from the even one's sum
+                float ss = 0.f;
 #pragma unroll
-            for (int i = 0; i < DPT; i++) x[i] = 0.f;
-        }
-        if (nw) {
-            float ss = 0.f;
+                for (int i = 0; i < DPT; i++) ss = fmaf(x[i], x[i], ss);
+                ss = __shfl_xor(ss, 1);
 #pragma unroll
-            for (int i = 0; i < DPT; i++) ss = fmaf(x[i], x[i], ss);
-            ss += __shfl_xor(ss, 1);
-            ss += __shfl_xor(ss, 2);
-            const float inv = tok >= 0 ? 1.0f / sqrtf(ss / (float)HD + eps) : 0.f;
+                for (int i = 0; i < DPT; i++) ss = fmaf(x[i], x[i], ss);
+                ss = __shfl(ss, (t & 63) | 1);
+                ss += __shfl_xor(ss, 2);
+                ss += __shfl_xor(ss, 4);
+                inv = tok >= 0 ? 1.0f / sqrtf(ss / (float)HD + eps) : 0.f;
 #pragma unroll
-            for (int i = 0; i < DPT; i++) x[i] = x[i] * inv * nw[d0 + i];
-        }
-        if (cosb) {
-            __syncthreads();
+                for (int i = 0; i < C4; i++) {
+                    const f32x4 w = *(const f32x4 *)&nw[d0 + 4 * i];
 #pragma unroll
-            for (int i = 0; i < DPT; i++) sx[r][d0 + i] = x[i];
-            __syncthreads();
-            // rot through an empty asm: otherwise the per-element region
-            // tests below are hoisted out of the q/k loop and their 64-bit
-            // lane masks, two per element, overflow the scalar registers
-            int rv = rot;
-            asm volatile("" : "+s"(rv));
-            const int half = rv >> 1;
-            if (tok >= 0 && (rv & 7) == 0) {
-                // 4-element chunks never straddle half or rot: one region
-                // test, and 16-byte reads of the tables and the partner chunk
-                const float *cr = cosb + (size_t)tok * rv, *sr = sinb + (size_t)tok * rv;
+                    for (int e = 0; e < 4; e++) x[4 * i + e] = x[4 * i + e] * inv * w[e];
+                }
+            }
+            if (rope4) {
+                if (tok >= 0) {
 #pragma unroll
-                for (int i = 0; i < DPT / 4; i++) {
-                    const int d = d0 + 4 * i;
-                    if (d < rv) {
-                        const bool lo = d < half;
-                        const f32x4 cv = *(const f32x4 *)(cr + d), sv = *(const f32x4 *)(sr + d);
-                        const f32x4 pv = *(const f32x4 *)&sx[r][lo ? d + half : d - half];
+                    for (int i = 0; i < C4; i++) {
+                        const int d = d0 + 4 * i;
+                        if (d < rot) {
+                            const bool lo = d < half;
+                            const int pd = lo ? d + half : d - half;
+                            f32x4 pv = *(const f32x4 *)&sx[prep_at<HD>(r, pd)];
+                            if (norm) {
+                                const f32x4 w = *(const f32x4 *)&nw[pd];
 #pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const float a = x[4 * i + e] * cv[e], b = pv[e] * sv[e];
-                            x[4 * i + e] = lo ? a - b : a + b;
+                                for (int e = 0; e < 4; e++) pv[e] = pv[e] * inv * w[e];
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                const float a = x[4 * i + e] * ct[i][e], b = pv[e] * st[i][e];
+                                x[4 * i + e] = lo ? a - b : a + b;
+                            }
                         }
                     }
                 }
-            } else if (tok >= 0) {
-                const float *cr = cosb + (size_t)tok * rv, *sr = sinb + (size_t)tok * rv;
+            } else if (ANYROT && tok >= 0) {
+                const float *cr = cosb + (size_t)tok * rot, *sr = sinb + (size_t)tok * rot;
+                // rot through an empty asm: otherwise the per-element region
+                // tests are hoisted out of the loops and their 64-bit lane
+                // masks, two per element, overflow the scalar registers
+                int rv = rot;
+                asm volatile("" : "+s"(rv));
+                const int hv = rv >> 1;
 #pragma unroll
                 for (int i = 0; i < DPT; i++) {
                     const int d = d0 + i;
-                    if (d < half) {
-                        const float a = x[i] * cr[d], b = sx[r][d + half] * sr[d];
-                        x[i] = a - b;
-                    } else if (d < rv) {
-                        const float a = x[i] * cr[d], b = sx[r][d - half] * sr[d];
-                        x[i] = a + b;
+                    if (d < rv) {
+                        const bool lo = d < hv;
+                        const int pd = lo ? d + hv : d - hv;
+                        float pv = sx[prep_at<HD>(r, pd)];
+                        if (norm) pv = pv * inv * nw[pd];
+                        const float a = x[i] * cr[d], b = pv * sr[d];
+                        x[i] = lo ? a - b : a + b;
                     }
                 }
             }
-        }
-        const int tile = blockIdx.x;
-        if (pl.q && tile < pl.T) {  // uniform over the workgroup
-            __syncthreads();
+            if (pl.q && tile < pl.T) {  // uniform over the workgroup
+                __syncthreads();
 #pragma unroll
-            for (int i = 0; i < DPT; i++) sx[r][d0 + i] = x[i];
-            __syncthreads();
-            pool_rows<HD>(sx, pl.cnt[tile], pl.inv[tile], (which ? pl.k : pl.q) + ((size_t)h * pl.T + tile) * HD);
-        }
-        if (!which) {
+                for (int i = 0; i < C4; i++)
+                    *(f32x4 *)&sx[prep_at<HD>(r, d0) + 4 * i] =
+                        f32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
+                __syncthreads();
+                pool_rows<HD>(sx, pl.cnt[tile], pl.inv[tile], (which ? pl.k : pl.q) + ((size_t)h * pl.T + tile) * HD);
+            }
+            const float sc = which ? 1.f : qscale;
+            half8 o[DPT / 8];
 #pragma unroll
-            for (int i = 0; i < DPT; i++) x[i] *= qscale;
+            for (int i = 0; i < DPT; i++) o[i / 8][i % 8] = (_Float16)(x[i] * sc);
+            half8 *dst = (half8 *)((which ? Kp : Qp) + ((size_t)h * n_pad + tile * ATT_PREP_T + r) * HD);
+            if constexpr (HD == 128) {
+                int at[2];
+                pair_chunks(o, c, at);
+                dst[at[0]] = o[0], dst[at[1]] = o[1];
+            } else {
+                dst[c] = o[0];
+            }
         }
-        half8 *dst = (half8 *)((which ? Kp : Qp) + ((size_t)h * n_pad + slot) * HD + d0);
+        // v: written transposed in the order above, four lanes to 64 bytes of a channel's row
+        if (pl.v && tile < pl.T)
+            pool_rows<HD>(sx, pl.cnt[tile], pl.inv[tile], pl.v + ((size_t)h * pl.T + tile) * HD);
+        int tv = t;
+        asm volatile("" : "+v"(tv));  // as in load()
 #pragma unroll
-        for (int i = 0; i < DPT / 8; i++) {
+        for (int i = 0; i < HD / 64; i++) {
+            const int id = tv + 512 * i, d = (id >> 2) % HD, j = id & 3, half_tile = id / (4 * HD);
+            // slots 32 half_tile + 8 j + e hold the keys that order names: row + (e % 4) + 2 (e & 4)
+            const int row = 32 * half_tile + 16 * (j >> 1) + 4 * (j & 1);
             half8 o;
 #pragma unroll
-            for (int e = 0; e < 8; e++) o[e] = (_Float16)x[8 * i + e];
-            dst[i] = o;
+            for (int e = 0; e < 8; e++) o[e] = (_Float16)sx[prep_at<HD>(row + (e & 3) + 2 * (e & 4), d)];
+            *(half8 *)(Vt + ((size_t)h * HD + d) * n_pad + (size_t)tile * ATT_PREP_T + 32 * half_tile + 8 * j) = o;
         }
     }
+}
 
-    // v: through LDS, written transposed in the vt_key order
-    __syncthreads();
-    if (tok >= 0) {
-        const f32x4 *p = (const f32x4 *)(v + (size_t)tok * ldv + (size_t)h * HD + d0);
-#pragma unroll
-        for (int i = 0; i < DPT / 4; i++) {
-            const f32x4 u = p[i];
-#pragma unroll
-            for (int e = 0; e < 4; e++) sx[r][d0 + 4 * i + e] = u[e];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < DPT; i++) sx[r][d0 + i] = 0.f;
-    }
-    __syncthreads();
-    if (pl.v && blockIdx.x < pl.T)
-        pool_rows<HD>(sx, pl.cnt[blockIdx.x], pl.inv[blockIdx.x], pl.v + ((size_t)h * pl.T + blockIdx.x) * HD);
-    constexpr int PER = ATT_PREP_T * HD / 256;  // slots written per thread (32 or 16)
-    constexpr int GROUPS = ATT_PREP_T / PER;
-    const int d = t / GROUPS, p0 = (t % GROUPS) * PER;
-    half8 *dst = (half8 *)(Vt + ((size_t)h * HD + d) * n_pad + (size_t)blockIdx.x * ATT_PREP_T + p0);
-#pragma unroll
-    for (int i = 0; i < PER / 8; i++) {
-        half8 o;
-#pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = (_Float16)sx[vt_key(p0 + 8 * i + e)][d];
-        dst[i] = o;
-    }
+// Heads per workgroup: up to four share a tile's table values while 2048
+// workgroups remain (eight to a CU).  n = 16384 x 40 heads: one 370, four 297,
+// eight 305 us; n = 1500 x 40, where it is one: 26.9, no faster with more.
+int prep_heads(int tiles, int heads) {
+    const int64_t g = (int64_t)tiles * heads / 2048;
+    return g < 1 ? 1 : g > 4 ? 4 : (int)g;
 }
 
 __device__ __forceinline__ float wave_swap_max(float x) { return fmaxf(x, __shfl_xor(x, 32)); }
@@ -408,8 +499,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
                 for (int v = 0; v < 16; v++) s[st][v] = __builtin_amdgcn_exp2f(s[st][v]);
 
             // P^T fragments: 16-key step t = values 4g..4g+7 of accumulator
-            // t/2, g = 2 (t % 2); they pair with V^T stored in the vt_key
-            // order.  The row sum is taken over the same fp16 values the
+            // t/2, g = 2 (t % 2); they pair with V^T stored in the order
+            // given above.  The row sum is taken over the same fp16 values the
             // product uses.
             half8 pf[4];
             float ps[2] = {0.f, 0.f};
@@ -677,8 +768,9 @@ hipError_t attn_launch(const float *q, const float *k, const float *v, int64_t l
     _Float16 *Kp = Qp + (size_t)heads * n_pad * HD;
     _Float16 *Vt = Kp + (size_t)heads * n_pad * HD;
     const float qscale = 1.4426950408889634f / sqrtf((float)HD);
-    hipLaunchKernelGGL(k_attn_prep<HD>, dim3(n_pad / ATT_PREP_T, heads), dim3(256), 0, st, q, k, v, ld, ld, n,
-                       (const int *)nullptr, qn_w, kn_w, eps, cosb, sinb, rot, qscale, n_pad, Qp, Kp, Vt, Pool{});
+    const int G = prep_heads(n_pad / ATT_PREP_T, heads);
+    hipLaunchKernelGGL((cosb && rot % 8 ? k_attn_prep<HD, true> : k_attn_prep<HD, false>),
+                       dim3(n_pad / ATT_PREP_T, (heads + G - 1) / G), dim3(512), 0, st, q, k, v, ld, ld, n, heads, G, (const int *)nullptr, qn_w, kn_w, eps, cosb, sinb, rot, qscale, n_pad, Qp, Kp, Vt, Pool{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     constexpr int NW = dense_nw(HD);
@@ -758,8 +850,10 @@ hipError_t vsa_launch(const float *q, const float *k, const float *v, int64_t ld
     VsaWs w = vsa_ws(ws, T, heads, HD);
     const float qscale = 1.4426950408889634f / sqrtf((float)HD);
     Pool pl{inv, cnt, w.qp, w.kp, gate ? w.vp : nullptr, T};
-    hipLaunchKernelGGL(k_attn_prep<HD>, dim3(n_pad / ATT_PREP_T, heads), dim3(256), 0, st, q, k, v, ld, ldv,
-                       ATT_KT * T, gather, qn_w, kn_w, eps, cosb, sinb, rot, qscale, n_pad, w.Qp, w.Kp, w.Vt, pl);
+    const int G = prep_heads(n_pad / ATT_PREP_T, heads);
+    hipLaunchKernelGGL((cosb && rot % 8 ? k_attn_prep<HD, true> : k_attn_prep<HD, false>),
+                       dim3(n_pad / ATT_PREP_T, (heads + G - 1) / G), dim3(512), 0, st, q, k, v, ld, ldv, ATT_KT * T,
+                       heads, G, gather, qn_w, kn_w, eps, cosb, sinb, rot, qscale, n_pad, w.Qp, w.Kp, w.Vt, pl);
     hipLaunchKernelGGL((k_vsa_scores<HD>), dim3(T, heads), dim3(256), 0, st, w.qp, w.kp, T, scale, w.sc);
     hipLaunchKernelGGL(k_vsa_lists, dim3(nqb, heads), dim3(256), (size_t)align256(6 * (size_t)T), st, w.sc, T, P, kv,
                        all, nqb, w.lists, w.list_len);
