@@ -577,181 +577,192 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
 // ---------------------------------------------------------------------------
 
 // scores[h][i][j] = (sum_d qp[h][i][d] * kp[h][j][d], in order) * scale
+// 64 x 64 tiles from LDS, 4 x 4 of them to a thread (rows and columns 16
+// apart: the eight lanes of a 16-byte LDS read then start on different banks).
+// Bound by the separate products and sums; 245 tiles x 56 heads: 194 -> 36 us
+// (before: every dot product read its whole key row from memory).
 template <int HD>
 __global__ __launch_bounds__(256) void k_vsa_scores(const float *__restrict__ qp, const float *__restrict__ kp,
                                                     int T, float scale, float *__restrict__ sc) {
-    __shared__ float qrow[HD];
-    const int i = blockIdx.x, h = blockIdx.y;
-    if (threadIdx.x < HD) qrow[threadIdx.x] = qp[((size_t)h * T + i) * HD + threadIdx.x];
-    __syncthreads();
-    for (int j = threadIdx.x; j < T; j += blockDim.x) {
-        const float *kr = kp + ((size_t)h * T + j) * HD;
-        float dot = 0.f;
-        for (int d = 0; d < HD; d++) dot = dot + qrow[d] * kr[d];
-        sc[((size_t)h * T + i) * T + j] = dot * scale;
+    __shared__ __align__(16) float sq[64][HD + 4], sk[64][HD + 4];
+    const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64, h = blockIdx.z, t = threadIdx.x;
+    for (int c = t; c < 64 * HD / 4; c += 256) {
+        const int r = c / (HD / 4), d = 4 * (c % (HD / 4));
+        const int i = i0 + r < T ? i0 + r : T - 1, j = j0 + r < T ? j0 + r : T - 1;
+        *(f32x4 *)&sq[r][d] = *(const f32x4 *)(qp + ((size_t)h * T + i) * HD + d);
+        *(f32x4 *)&sk[r][d] = *(const f32x4 *)(kp + ((size_t)h * T + j) * HD + d);
     }
+    __syncthreads();
+    const int ti = t >> 4, tj = t & 15;
+    float dot[4][4] = {};
+#pragma unroll 4
+    for (int d = 0; d < HD; d += 4) {
+        f32x4 a[4], b[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            a[x] = *(const f32x4 *)&sq[ti + 16 * x][d];
+            b[x] = *(const f32x4 *)&sk[tj + 16 * x][d];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+#pragma unroll
+                for (int y = 0; y < 4; y++) dot[x][y] = dot[x][y] + a[x][e] * b[y][e];
+    }
+#pragma unroll
+    for (int x = 0; x < 4; x++)
+#pragma unroll
+        for (int y = 0; y < 4; y++) {
+            const int i = i0 + ti + 16 * x, j = j0 + tj + 16 * y;
+            if (i < T && j < T) sc[((size_t)h * T + i) * T + j] = dot[x][y] * scale;
+        }
 }
 
-// The selection of query tile i as flags sel[j] (LDS): every tile for prefix
-// query tiles or when all are kept; otherwise the prefix tiles and the kv
-// video tiles of largest score, ties to the lower tile index (the order of
-// the reference's qsort comparator, src/core/fh3_vsa.c:178-184).  The kv-th
-// largest score is found by a 4-pass radix select on order-preserving keys.
-__device__ void vsa_select_row(const float *__restrict__ srow, int T, int P, int kv, bool all, int i,
-                               uint32_t *keys, uint8_t *sel, int *hist, int *scal) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    if (i < P || all) {
-        for (int j = tid; j < T; j += nt) sel[j] = 1;
-        __syncthreads();
-        return;
-    }
-    const int NV = T - P;
-    for (int j = tid; j < T; j += nt) {
-        sel[j] = j < P;
-        if (j >= P) {
+// The selection of one query tile by one wavefront, as bits m[e] of the key
+// tiles 64 e + lane: every tile for prefix query tiles or when all are kept;
+// otherwise the prefix tiles and the kv video tiles of largest score, ties to
+// the lower tile index (the order of the reference's qsort comparator,
+// src/core/fh3_vsa.c:178-184).  The scores become order-preserving keys, held in
+// registers; the kv-th largest is built bit by bit, each bit kept where at least
+// kv keys reach it.
+template <int R>
+__device__ __forceinline__ void vsa_select_row(const float *__restrict__ srow, int T, int P, int kv, bool all,
+                                               uint64_t (&m)[R]) {
+    const int lane = threadIdx.x & 63;
+    uint32_t key[R];
+#pragma unroll
+    for (int e = 0; e < R; e++) {
+        const int j = 64 * e + lane;
+        m[e] = __ballot(j < T && (all || j < P));
+        key[e] = 0;  // below every threshold tried
+        if (!all && j >= P && j < T) {
             float f = srow[j];
             f = f == 0.f ? 0.f : f;  // -0 ties with +0, as in the comparator
             const uint32_t u = __float_as_uint(f);
-            keys[j - P] = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+            key[e] = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
         }
     }
-    uint32_t prefix = 0, mask = 0;
-    int want = kv;
-    for (int pass = 0; pass < 4; pass++) {
-        const int shift = 24 - 8 * pass;
-        for (int b = tid; b < 256; b += nt) hist[b] = 0;
-        __syncthreads();
-        for (int j = tid; j < NV; j += nt)
-            if ((keys[j] & mask) == prefix) atomicAdd(&hist[(keys[j] >> shift) & 255], 1);
-        __syncthreads();
-        if (tid == 0) {
-            int above = 0, b = 255;
-            for (; b > 0; b--) {
-                if (above + hist[b] >= want) break;
-                above += hist[b];
-            }
-            scal[0] = b;
-            scal[1] = want - above;
-        }
-        __syncthreads();
-        prefix |= (uint32_t)scal[0] << shift;
-        mask |= 0xFFu << shift;
-        want = scal[1];
-        __syncthreads();
+    if (all) return;
+    uint32_t thr = 0;
+    for (int bit = 31; bit >= 0; bit--) {
+        const uint32_t cand = thr | (1u << bit);
+        int cnt = 0;
+#pragma unroll
+        for (int e = 0; e < R; e++) cnt += (int)__popcll(__ballot(key[e] >= cand));
+        if (cnt >= kv) thr = cand;
     }
-    // keys above the threshold are in; of those equal to it, the first `want`
-    // by tile index (a block-wide running count over j in order)
-    if (tid == 0) scal[2] = 0;
-    __syncthreads();
-    for (int j0 = 0; j0 < NV; j0 += nt) {
-        const int j = j0 + tid;
-        const bool eq = j < NV && keys[j] == prefix;
-        const uint64_t bal = __ballot(eq);
-        const int wave = tid >> 6, lane = tid & 63;
-        if (lane == 0) hist[wave] = __popcll(bal);
-        __syncthreads();
-        int before = scal[2];
-        for (int w = 0; w < wave; w++) before += hist[w];
-        before += __popcll(bal & ((lane ? (~0ull >> (64 - lane)) : 0ull)));
-        if (j < NV) sel[P + j] = keys[j] > prefix || (eq && before < want);
-        __syncthreads();
-        if (tid == 0) {
-            int tot = 0;
-            for (int w = 0; w < (nt >> 6); w++) tot += hist[w];
-            scal[2] += tot;
-        }
-        __syncthreads();
+    int want = kv;  // how many of the keys equal to the threshold are in
+#pragma unroll
+    for (int e = 0; e < R; e++) want -= (int)__popcll(__ballot(key[e] > thr));
+#pragma unroll
+    for (int e = 0; e < R; e++) {
+        const int j = 64 * e + lane;
+        const uint64_t eq = __ballot(j >= P && j < T && key[e] == thr);
+        const bool in = key[e] > thr || (((eq >> lane) & 1) && (int)__popcll(eq & ((1ull << lane) - 1)) < want);
+        m[e] |= __ballot(in);
+        want -= (int)__popcll(eq);
     }
 }
 
-// Union tile lists of query-tile pairs (2 qb, 2 qb + 1) for k_attn_fwd.
-__global__ __launch_bounds__(256) void k_vsa_lists(const float *__restrict__ sc, int T, int P, int kv, int all,
+// Union tile lists of query-tile pairs (2 qb, 2 qb + 1) for k_attn_fwd: a
+// wavefront selects for each of the two, the first writes the list in tile
+// order.  T <= 64 R.  245 tiles x 56 heads: 229 -> 16 us (before: a radix select
+// over LDS histograms that one thread scanned).
+template <int R>
+__global__ __launch_bounds__(128) void k_vsa_lists(const float *__restrict__ sc, int T, int P, int kv, int all,
                                                    int nqb, uint16_t *__restrict__ lists,
                                                    int *__restrict__ list_len) {
-    extern __shared__ uint8_t smem[];
-    uint32_t *keys = (uint32_t *)smem;                    // [T]
-    uint8_t *sel0 = smem + (size_t)4 * T, *sel1 = sel0 + T;
-    __shared__ int hist[256];
-    __shared__ int scal[4];
-    const int qb = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, nt = blockDim.x;
-    const int i0 = 2 * qb, i1 = 2 * qb + 1;
-    vsa_select_row(sc + ((size_t)h * T + i0) * T, T, P, kv, all != 0, i0, keys, sel0, hist, scal);
-    if (i1 < T) {
-        vsa_select_row(sc + ((size_t)h * T + i1) * T, T, P, kv, all != 0, i1, keys, sel1, hist, scal);
-    } else {
-        for (int j = tid; j < T; j += nt) sel1[j] = 0;
-        __syncthreads();
+    __shared__ uint64_t sel1[R];
+    const int qb = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = 2 * qb + wave;
+    uint64_t m[R] = {};
+    if (i < T) vsa_select_row<R>(sc + ((size_t)h * T + i) * T, T, P, kv, all != 0 || i < P, m);
+    if (wave == 1 && lane == 0) {
+#pragma unroll
+        for (int e = 0; e < R; e++) sel1[e] = m[e];
     }
-    // stream compaction in tile order
-    uint16_t *out = lists + ((size_t)h * nqb + qb) * T;
-    if (tid == 0) scal[3] = 0;
     __syncthreads();
-    for (int j0 = 0; j0 < T; j0 += nt) {
-        const int j = j0 + tid;
-        const int bits = j < T ? (sel0[j] ? 1 : 0) | (sel1[j] ? 2 : 0) : 0;
-        const uint64_t bal = __ballot(bits != 0);
-        const int wave = tid >> 6, lane = tid & 63;
-        if (lane == 0) hist[wave] = __popcll(bal);
-        __syncthreads();
-        int at = scal[3];
-        for (int w = 0; w < wave; w++) at += hist[w];
-        at += __popcll(bal & ((lane ? (~0ull >> (64 - lane)) : 0ull)));
-        if (bits) out[at] = (uint16_t)(j | (bits << 14));
-        __syncthreads();
-        if (tid == 0) {
-            int tot = 0;
-            for (int w = 0; w < (nt >> 6); w++) tot += hist[w];
-            scal[3] += tot;
-        }
-        __syncthreads();
+    if (wave == 1) return;
+    uint16_t *out = lists + ((size_t)h * nqb + qb) * T;
+    int at = 0;
+#pragma unroll
+    for (int e = 0; e < R; e++) {
+        const uint64_t b = sel1[e], u = m[e] | b;
+        const int bits = (int)((m[e] >> lane) & 1) | (int)((b >> lane) & 1) << 1;
+        if (bits) out[at + __popcll(u & ((1ull << lane) - 1))] = (uint16_t)((64 * e + lane) | (bits << 14));
+        at += __popcll(u);
     }
-    if (tid == 0) list_len[h * nqb + qb] = scal[3];
+    if (lane == 0) list_len[h * nqb + qb] = at;
 }
 
 // Gated coarse branch: per (query tile i, head h) a softmax over all tile
 // scores mixes the pooled v: coarse[h][i][d] = sum_j expf(s_j - max) / sum * vp[h][j][d].
-template <int HD>
+// A workgroup takes RB query tiles, so that each pooled v is read once for all of
+// them: 245 tiles x 56 heads 84 -> 47 us.
+template <int HD, int RB>
 __global__ __launch_bounds__(HD) void k_vsa_coarse(const float *__restrict__ sc, const float *__restrict__ vp,
                                                    int T, float *__restrict__ coarse) {
-    extern __shared__ float wsh[];  // [T] softmax weights
-    __shared__ float red[HD / 64];
-    __shared__ float bc[2];
-    const int i = blockIdx.x, h = blockIdx.y, d = threadIdx.x, lane = d & 63, wave = d >> 6;
-    const float *srow = sc + ((size_t)h * T + i) * T;
-    float mx = -1e30f;
-    for (int j = d; j < T; j += HD) mx = fmaxf(mx, srow[j]);
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if (lane == 0) red[wave] = mx;
-    __syncthreads();
-    if (d == 0) {
-        float m = red[0];
-        for (int w = 1; w < HD / 64; w++) m = fmaxf(m, red[w]);
-        bc[0] = m;
+    extern __shared__ __align__(16) float wsh[];  // [T][RB] softmax weights
+    __shared__ float red[RB][HD / 64];
+    const int i0 = blockIdx.x * RB, h = blockIdx.y, d = threadIdx.x, lane = d & 63, wave = d >> 6;
+    const float *srow[RB];
+    float mx[RB], sum[RB], acc[RB];
+#pragma unroll
+    for (int x = 0; x < RB; x++) {
+        srow[x] = sc + ((size_t)h * T + (i0 + x < T ? i0 + x : T - 1)) * T;
+        mx[x] = -1e30f;
+        sum[x] = acc[x] = 0.f;
+    }
+    for (int j = d; j < T; j += HD)
+#pragma unroll
+        for (int x = 0; x < RB; x++) mx[x] = fmaxf(mx[x], srow[x][j]);
+#pragma unroll
+    for (int x = 0; x < RB; x++) {
+        for (int o = 32; o > 0; o >>= 1) mx[x] = fmaxf(mx[x], __shfl_xor(mx[x], o));
+        if (lane == 0) red[x][wave] = mx[x];
     }
     __syncthreads();
-    mx = bc[0];
-    float sum = 0.f;
-    for (int j = d; j < T; j += HD) {
-        wsh[j] = expf(srow[j] - mx);
-        sum += wsh[j];
+#pragma unroll
+    for (int x = 0; x < RB; x++) {
+        mx[x] = red[x][0];
+        for (int w = 1; w < HD / 64; w++) mx[x] = fmaxf(mx[x], red[x][w]);
     }
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-    __syncthreads();
-    if (lane == 0) red[wave] = sum;
-    __syncthreads();
-    if (d == 0) {
-        float t = 0.f;
-        for (int w = 0; w < HD / 64; w++) t += red[w];
-        bc[1] = 1.0f / t;
+    for (int j = d; j < T; j += HD)
+#pragma unroll
+        for (int x = 0; x < RB; x++) {
+            const float w = expf(srow[x][j] - mx[x]);
+            wsh[j * RB + x] = w;
+            sum[x] += w;
+        }
+    __syncthreads();  // red is read
+#pragma unroll
+    for (int x = 0; x < RB; x++) {
+        for (int o = 32; o > 0; o >>= 1) sum[x] += __shfl_xor(sum[x], o);
+        if (lane == 0) red[x][wave] = sum[x];
     }
     __syncthreads();
-    const float inv = bc[1];
-    for (int j = d; j < T; j += HD) wsh[j] = wsh[j] * inv;
+#pragma unroll
+    for (int x = 0; x < RB; x++) {
+        sum[x] = 0.f;
+        for (int w = 0; w < HD / 64; w++) sum[x] += red[x][w];
+        sum[x] = 1.0f / sum[x];
+    }
+    for (int j = d; j < T; j += HD)
+#pragma unroll
+        for (int x = 0; x < RB; x++) wsh[j * RB + x] = wsh[j * RB + x] * sum[x];
     __syncthreads();
-    float acc = 0.f;
     const float *vcol = vp + (size_t)h * T * HD + d;
-    for (int j = 0; j < T; j++) acc += wsh[j] * vcol[(size_t)j * HD];
-    coarse[((size_t)h * T + i) * HD + d] = acc;
+#pragma unroll 4
+    for (int j = 0; j < T; j++) {
+        const float v = vcol[(size_t)j * HD];
+#pragma unroll
+        for (int x = 0; x < RB; x++) acc[x] += wsh[j * RB + x] * v;
+    }
+#pragma unroll
+    for (int x = 0; x < RB; x++)
+        if (i0 + x < T) coarse[((size_t)h * T + i0 + x) * HD + d] = acc[x];
 }
 
 int64_t attn_pad_dense(int n, int hd) {
@@ -854,12 +865,16 @@ hipError_t vsa_launch(const float *q, const float *k, const float *v, int64_t ld
     hipLaunchKernelGGL((cosb && rot % 8 ? k_attn_prep<HD, true> : k_attn_prep<HD, false>),
                        dim3(n_pad / ATT_PREP_T, (heads + G - 1) / G), dim3(512), 0, st, q, k, v, ld, ldv, ATT_KT * T,
                        heads, G, gather, qn_w, kn_w, eps, cosb, sinb, rot, qscale, n_pad, w.Qp, w.Kp, w.Vt, pl);
-    hipLaunchKernelGGL((k_vsa_scores<HD>), dim3(T, heads), dim3(256), 0, st, w.qp, w.kp, T, scale, w.sc);
-    hipLaunchKernelGGL(k_vsa_lists, dim3(nqb, heads), dim3(256), (size_t)align256(6 * (size_t)T), st, w.sc, T, P, kv,
-                       all, nqb, w.lists, w.list_len);
-    if (gate)
-        hipLaunchKernelGGL((k_vsa_coarse<HD>), dim3(T, heads), dim3(HD), (size_t)T * sizeof(float), st, w.sc, w.vp, T,
-                           w.coarse);
+    const int t64 = (T + 63) / 64;
+    hipLaunchKernelGGL((k_vsa_scores<HD>), dim3(t64, t64, heads), dim3(256), 0, st, w.qp, w.kp, T, scale, w.sc);
+    hipLaunchKernelGGL((T <= 256 ? k_vsa_lists<4> : T <= 1024 ? k_vsa_lists<16> : k_vsa_lists<64>), dim3(nqb, heads),
+                       dim3(128), 0, st, w.sc, T, P, kv, all, nqb, w.lists, w.list_len);
+    if (gate) {
+        // eight query tiles to a workgroup while their weights take at most 32 KB of LDS
+        const int rb = T <= 1024 ? 8 : 2;
+        hipLaunchKernelGGL((rb == 8 ? k_vsa_coarse<HD, 8> : k_vsa_coarse<HD, 2>), dim3((T + rb - 1) / rb, heads),
+                           dim3(HD), (size_t)T * rb * sizeof(float), st, w.sc, w.vp, T, w.coarse);
+    }
     Sparse sp{w.lists, w.list_len, cnt, gather, gate ? w.coarse : nullptr, gate, T};
     hipLaunchKernelGGL((k_attn_fwd<HD, true, ATT_NW>), dim3(heads * nqb), dim3(64 * ATT_NW), 0, st, w.Qp, w.Kp, w.Vt,
                        ATT_KT * T, n_pad, heads, o, o_ld, sp);
