@@ -805,6 +805,13 @@ static int matmul_dev(const Fh3W *w, const float *d_x, float *d_y, int n_tok, co
     rc = ensure_init();
     if (rc != FH3_OK) return rc;
     hipStream_t st = stream ? (hipStream_t)stream : g.stream;
+    if (w->type == FH3_QUANT_F16 && g.path == FH3_HIP_PATH_AUTO && w->in <= 128 &&
+        fh3k_short16_fits((int)w->in, (int)w->out, n_tok)) {
+        // no preparation and no workspace; longer rows, whose operands no longer fit one workgroup, take
+        // the general route below (at its shortest of 128: 10-191 us for 1-16384 tokens against 6-89 here)
+        FH3_HIPCALL(fh3k_short16(w->data, (int)w->out, (int)w->in, d_x, d_bias_or_null, d_y, n_tok, st));
+        return FH3_OK;
+    }
     if (w->type != FH3_QUANT_Q4_K || general_rows(w->in)) {
         std::lock_guard<std::recursive_mutex> lk(g.mu);
         const int64_t rows = path16(n_tok, w->in) == FH3_HIP_PATH_SKINNY ? round_up(n_tok, 32) : prep_rows(n_tok);

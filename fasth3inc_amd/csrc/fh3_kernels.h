@@ -63,6 +63,10 @@ hipError_t fh3k_skinny16(const void *W16, int N, int K, const void *x16, const f
                          float *y, int M, hipStream_t st);
 hipError_t fh3k_gemm16(const void *W16, int N, int K, const void *x16, const float *xs_inv, const float *bias,
                        float *y, int M, hipStream_t st);
+// Short F16 rows straight from fp32 activations, in one launch.
+int fh3k_short16_fits(int K, int N, int M);
+hipError_t fh3k_short16(const void *W16, int N, int K, const float *x, const float *bias, float *y, int M,
+                        hipStream_t st);
 // Q5_K / Q6_K weights (type FH3K_Q5_K / FH3K_Q6_K) read in place by the
 // small-M kernel, M <= fh3k_skinny_max_tokens(), same fragments as fh3k_skinny;
 // fh3k_skinny_q_takes(type) says whether a type has this kernel.  Rows that

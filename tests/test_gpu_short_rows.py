@@ -1,0 +1,45 @@
+"""Short F16 rows in one launch (k_short16) against the general route, which a
+forced path still takes: the same bits, non-finite activations included, at the
+edges of its 128 x 128 tiles and of its row lengths (8 to 128 by 8; 136 is past it)."""
+import numpy as np
+import pytest
+
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K,N,bias", [(1, 8, 1, True), (3, 96, 5376, True), (64, 32, 127, False),
+                                        (65, 24, 129, True), (127, 128, 128, True), (128, 104, 257, False),
+                                        (129, 96, 31, True), (300, 120, 1000, True), (2880, 96, 5376, True),
+                                        (130, 136, 130, True)])
+def test_short_rows_same_bits(gpu, M, K, N, bias):
+    F = gpu
+    print("short rows M=%d K=%d N=%d" % (M, K, N), flush=True)
+    rng = np.random.default_rng(M + K + N)
+    w = rng.standard_normal((N, K)).astype(np.float16)
+    x = rng.standard_normal((M, K)).astype(np.float32) * np.exp2(rng.integers(-20, 20, (M, 1))).astype(np.float32)
+    if M > 2:
+        x[1] = 0
+        x[2, K // 2] = np.inf
+    if M > 64:
+        x[M - 1, 0] = np.nan
+    b = rng.standard_normal(N).astype(np.float32) if bias else None
+    bufs = [F.DeviceBuffer.from_array(a) if a is not None else None for a in (w, x, b)]
+    out = []
+    for path in (F.PATH_AUTO, F.PATH_GEMM):
+        y = F.DeviceBuffer.from_array(np.full((M + 1) * N, 7, np.float32))
+        F.set_path(path)
+        try:
+            F.matmul_dev(bufs[0], K, N, bufs[1], y, M, bufs[2], qtype=F.FH3_QUANT_F16)
+            F.synchronize()
+        finally:
+            F.set_path(F.PATH_AUTO)
+        out.append(y.download(np.float32, (M + 1, N)))
+    assert (out[0][M] == 7).all()
+    nan = np.isnan(out[1])
+    assert np.array_equal(np.isnan(out[0]), nan)
+    assert np.array_equal(np.where(nan, 0, out[0]).view(np.uint32), np.where(nan, 0, out[1]).view(np.uint32))
+    ok = np.isfinite(x).all(1)
+    ref = x[ok].astype(np.float64) @ w.astype(np.float64).T + (0 if b is None else b)
+    assert H.rel_fro(out[0][:M][ok], ref) <= 1e-3  # one rounding of x to fp16 (2^-11) and fp32 sums
