@@ -273,22 +273,32 @@ __device__ __forceinline__ void deq_piece(const uint8_t *blk, int G, float o[16]
     }
 }
 
+// Sixteen outputs per thread, bound by their stores.  A thread's 64 bytes go
+// through LDS, so that each store of a wavefront covers 1024 consecutive bytes,
+// and past the caches.  Q6_K, 8192 x 5120: 63.9 us with 16-byte pieces 64 bytes
+// apart and a division for the row, 42.3 in order, 30.2 (6.7 TB/s) past the caches.
+// total: 16-value pieces of all rows, which follow one another without a gap.
 template <int T>
-__global__ __launch_bounds__(256) void k_dequant_blocks(const uint8_t *__restrict__ src, int64_t row_bytes,
-                                                        int64_t nblk, int64_t rows, float *__restrict__ dst) {
-    constexpr int BL = Fmt<T>::BL, BB = Fmt<T>::BB, P = Fmt<T>::P;
-    const int64_t per_row = nblk * P;
+__global__ __launch_bounds__(256) void k_dequant_blocks(const uint8_t *__restrict__ src, int64_t total,
+                                                        float *__restrict__ dst) {
+    constexpr int BB = Fmt<T>::BB, P = Fmt<T>::P;
+    __shared__ f32x4 so[4][4][68];  // [wavefront][quarter of its lanes][16 lanes x 4, padded]
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= rows * per_row) return;
-    const int64_t row = gid / per_row;
-    const int64_t rem = gid - row * per_row;
-    const int64_t b = rem / P;
-    const int G = (int)(rem - b * P);
-    float o[16];
-    deq_piece<T>(src + row * row_bytes + b * BB, G, o);
-    f32x4 *out = reinterpret_cast<f32x4 *>(dst + row * nblk * BL + b * BL + 16 * G);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (gid < total) {
+        float o[16];
+        deq_piece<T>(src + gid / P * BB, (int)(gid % P), o);
 #pragma unroll
-    for (int j = 0; j < 4; j++) out[j] = f32x4{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+        for (int j = 0; j < 4; j++)
+            so[wave][lane >> 4][(lane & 15) * 4 + j] = f32x4{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    f32x4 *out = reinterpret_cast<f32x4 *>(dst) + (gid - lane) * 4;
+    const int64_t left = (total - (gid - lane)) * 4;  // 16-byte pieces of this wavefront's outputs that exist
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (64 * i + lane < left) __builtin_nontemporal_store(so[wave][i][lane], out + 64 * i + lane);
 }
 
 // F16 (fh3_quant.c:36-49, exact, F16C NaN quieting) and BF16 (:51-56, the bits
@@ -2990,11 +3000,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm16(const _Float16 *__restrict__ 
 template <int T>
 static hipError_t launch_dequant_blocks(const void *src, int64_t row_bytes, int64_t n, int64_t rows, float *dst,
                                         hipStream_t st) {
-    const int64_t nblk = n / Fmt<T>::BL;
-    const int64_t blocks = (rows * nblk * Fmt<T>::P + 255) / 256;
-    if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_dequant_blocks<T>, dim3((unsigned)blocks), dim3(256), 0, st, (const uint8_t *)src,
-                       row_bytes, nblk, rows, dst);
+    const int64_t nblk = n / Fmt<T>::BL, total = rows * nblk * Fmt<T>::P;
+    const int64_t blocks = (total + 255) / 256;
+    if (blocks > 0x7FFFFFFF || (rows > 1 && row_bytes != nblk * Fmt<T>::BB)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_dequant_blocks<T>, dim3((unsigned)blocks), dim3(256), 0, st, (const uint8_t *)src, total,
+                       dst);
     return hipGetLastError();
 }
 
