@@ -2206,22 +2206,39 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         if constexpr (TBW == 1) return acc.v[v >> 3][2 * ob + ((v >> 2) & 1)][v & 3];
         else return acc.v[tb][ob][v];
     };
+    // The bias of a lane's columns of the block from column c0 (one, or two 16
+    // apart), read once per block: read for each value, the 16-byte-store paths held
+    // twice the loads and branches, and a call took 0.8 us longer (512 x 256 ->
+    // 5120 11.0 -> 11.8, now 11.0; SwiGLU 507 x 1024 -> 17408 39.0 -> 42.4, now 39.0).
+    struct Bias { float c[TBW == 1 ? 2 : 1]; };
+    auto block_bias = [&](int c0) {
+        Bias b;
+        b.c[0] = bias ? bias[c0 + vcol(0)] : 0.f;
+        if constexpr (TBW == 1) b.c[1] = bias ? bias[c0 + vcol(4)] : 0.f;
+        return b;
+    };
+    auto value_bias = [](const Bias &b, int v) { return b.c[TBW == 1 ? (v >> 2) & 1 : 0]; };
     // Fast path: a 32x32 block whose rows and 32 columns are all inside the
     // output (row stride a multiple of 4 floats) goes through this wavefront's
     // 4 KiB of LDS (free after the loop's last barrier) and leaves as 16-byte
     // row pieces: 4 vector stores per lane instead of 16 scalar ones (the
     // scalar stores cost ~7 % of the kernel on the DiT shapes).  Values and
-    // rounding are the same either way.
+    // rounding are the same either way.  With one token block the last tokens'
+    // partial blocks go the same way, `rows` of them: a scalar store covers only 64
+    // bytes of a row there (100 x 256 -> 5120: 10.0 us, now 7.0; blocks 32 wide
+    // had taken 8.8).
     float *stg = reinterpret_cast<float *>(&lds[0][0][0]) + wave * 1024;
-    // dst points at the block's top-left element, ld is the row stride;
+    // dst points at the block's top-left element, ld is the row stride, rows
+    // how many of the block's rows exist;
     // mode 0 store, 1 gate residual (dst += g * y, g at the same offsets in aux)
-    auto block_store = [&](const float (&val)[16], float *dst, const float *g, size_t ld, int mode) {
+    auto block_store = [&](const float (&val)[16], float *dst, const float *g, size_t ld, int mode, int rows) {
 #pragma unroll
         for (int v = 0; v < 16; v++) stg[vrow(v) * 32 + vcol(v)] = val[v];
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int r = (lane >> 3) + 8 * i, c = 4 * (lane & 7);
+            if (TBW == 1 && r >= rows) continue;
             const f32x4 y = *reinterpret_cast<const f32x4 *>(stg + r * 32 + c);
             f32x4 *d = reinterpret_cast<f32x4 *>(dst + (size_t)r * ld + c);
             if (mode == 1) {
@@ -2255,7 +2272,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
                     float vals[16];
 #pragma unroll
                     for (int v = 0; v < 16; v++) vals[v] = vacc(tb, ob, v);
-                    block_store(vals, part + ((size_t)ks * M + tb0) * N + c0, nullptr, (size_t)N, 0);
+                    block_store(vals, part + ((size_t)ks * M + tb0) * N + c0, nullptr, (size_t)N, 0, 32);
                 }
             }
             return;
@@ -2284,14 +2301,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
                 const int tb0 = wt0 + 32 * tb;
 #pragma unroll
                 for (int ob = 0; ob < 2; ob++) {
+                    const int c0 = nt * 64 + 32 * ob;
+                    const Bias bbv = block_bias(c0), bbg = block_bias(F + c0);
                     float vals[16];
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const int t = tb0 + vrow(v), o = nt * 64 + 32 * ob + vcol(v);
-                        const float bv = bias ? bias[o] : 0.f, bg = bias ? bias[F + o] : 0.f;
+                        const int t = tb0 + vrow(v);
+                        const float bv = value_bias(bbv, v), bg = value_bias(bbg, v);
                         vals[v] = (vacc(tb, ob, v) * xs_inv[t] + bv) * silu_f32(vacc(tb, ob + 2, v) * xs_inv[t] + bg);
                     }
-                    block_store(vals, Y + (size_t)tb0 * F + nt * 64 + 32 * ob, nullptr, (size_t)F, 0);
+                    block_store(vals, Y + (size_t)tb0 * F + nt * 64 + 32 * ob, nullptr, (size_t)F, 0, 32);
                 }
             }
             return;
@@ -2300,10 +2319,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         for (int tb = 0; tb < TBW; tb++) {
 #pragma unroll
             for (int ob = 0; ob < 2; ob++) {
+                const int c0 = nt * 64 + 32 * ob;
+                const Bias bbv = block_bias(c0), bbg = block_bias(F + c0);
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    const int t = wt0 + 32 * tb + vrow(v), o = nt * 64 + 32 * ob + vcol(v);
-                    const float bv = bias ? bias[o] : 0.f, bg = bias ? bias[F + o] : 0.f;
+                    const int t = wt0 + 32 * tb + vrow(v), o = c0 + vcol(v);
+                    const float bv = value_bias(bbv, v), bg = value_bias(bbg, v);
                     if (t < M)
                         Y[(size_t)t * F + o] = (vacc(tb, ob, v) * xs_inv[t] + bv) *
                                                silu_f32(vacc(tb, ob + 2, v) * xs_inv[t] + bg);
@@ -2312,19 +2333,20 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
         }
         return;
     }
-    if (rows_in && out16 && (N & 3) == 0 && n0 + 128 <= N) {
+    if ((TBW == 1 || rows_in) && out16 && (N & 3) == 0 && n0 + 128 <= N) {
 #pragma unroll
         for (int tb = 0; tb < TBW; tb++) {
             const int tb0 = wt0 + 32 * tb;
 #pragma unroll
             for (int ob = 0; ob < 4; ob++) {
+                const Bias bb = block_bias(n0 + 32 * ob);
                 float vals[16];
 #pragma unroll
                 for (int v = 0; v < 16; v++)
-                    vals[v] = vacc(tb, ob, v) * xs_inv[tb0 + vrow(v)] + (bias ? bias[n0 + 32 * ob + vcol(v)] : 0.f);
+                    vals[v] = vacc(tb, ob, v) * xs_inv[tb0 + vrow(v)] + value_bias(bb, v);
                 const size_t off = (size_t)tb0 * N + n0 + 32 * ob;
                 block_store(vals, Y + off, epi == EPI_GATE_RES ? aux + off : nullptr, (size_t)N,
-                            epi == EPI_GATE_RES ? 1 : 0);
+                            epi == EPI_GATE_RES ? 1 : 0, M - tb0);
             }
         }
         return;
