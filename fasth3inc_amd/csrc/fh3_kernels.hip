@@ -3864,26 +3864,34 @@ static hipError_t launch_gemm256(const void *W, int64_t row_bytes, int N, int K,
     return hipGetLastError();
 }
 
-// Estimated times of both forms in us at K = 5120 (they scale with K), from
-// rounds of the 256 CUs.  k_gemm: 157 us per full round of 512 tiles of 256 x
-// 128, 64 + 0.18 us per tile of the last one; k_gemm256: 119 us per full round
-// of 256, 105 for the last, and the decode, 2.56 bytes per weight at 5 TB/s.
-// Measured, k_gemm against both launches, us: K = 5120, N = 17408 at 1024 /
-// 1500 / 2048 / 3016 tokens 233 / 285 / 382 / 536 against 242 / 254 / 380 / 495;
-// N = 5120 at 2048 / 4096 / 8192 tokens 128 / 236 / 406 against 114 / 219 /
-// 343; N = 1024 / 2048 at 4096 tokens 86 / 101 against 93 / 105; 6000 tokens,
-// 1024 -> 2000 48 against 36.  Only where k_gemm does not split K: the two then
-// give the same bits, which one a call takes cannot be told from its result.
+// Estimated times of both forms in us, from their rounds of workgroups on the
+// 256 CUs (k_gemm 512 tiles of 256 x 128 a round, k_gemm256 256 of 256 x 256): a
+// part in K and a fixed one (prologue, epilogue; k_gemm256, one workgroup to a CU,
+// overlaps neither), the launches, the decode, and the scalar stores of rows
+// that are no multiple of 4 floats and of k_gemm's last columns.  Fitted to 673 shapes
+// (K 256-25600, N 1000-28672, 1024-32768 tokens, every type and epilogue) with both
+// forms timed: 7 / 5 % rms.  What they choose is 10.6 % faster than k_gemm alone
+// (geometric mean; 11.3 the better form each time), at worst 6 % slower at K >=
+// 1024; with times that only scaled with K (8.4 %) 96 of the shapes had become
+// slower: 2048 x 1024 -> 5120 31.6 -> 40.7 us, now 31.6; 2048 x 256 -> 5120 15.7 -> 24.6.
+// Only where k_gemm does not split K: the two then give the same bits, which one
+// a call takes cannot be told from its result.
 static bool gemm256_wins(int N, int K, int M, int epi) {
     int C, S;
     gemm_split(M, N, K, epi, C, S);
     if (M < 1024 || S > 1) return false;
     const int64_t mt = (M + 255) / 256;
-    const int64_t t0 = mt * (epi == EPI_SWIGLU ? (N / 2) / 64 : (N + GEMM_BN - 1) / GEMM_BN);
-    const int64_t t1 = mt * (epi == EPI_SWIGLU ? (N / 2 + 127) / 128 : (N + G256_B - 1) / G256_B);
-    const double one = t0 / 512 * 157.0 + (t0 % 512 ? 64.0 + 0.18 * (double)(t0 % 512) : 0.0);
-    const double two = t1 / 256 * 119.0 + (t1 % 256 ? 105.0 : 0.0) + (double)N * 5120.0 * 2.56 / 5.0e6;
-    return two < 0.98 * one;
+    const bool sw = epi == EPI_SWIGLU;
+    const int64_t t0 = mt * (sw ? (N / 2) / 64 : (N + GEMM_BN - 1) / GEMM_BN);
+    const int64_t t1 = mt * (sw ? (N / 2 + 127) / 128 : (N + G256_B - 1) / G256_B);
+    const int64_t f0 = t0 / 512, r0 = t0 % 512, f1 = t1 / 256, r1 = t1 % 256;
+    const double k = K / 5120.0, rounds0 = (double)(f0 + (r0 > 0)), rounds1 = (double)(f1 + (r1 > 0));
+    const bool scalar = (sw ? N / 2 : N) % 4 != 0, edge = !sw && !scalar && N % GEMM_BN;
+    const double one = 7.0 + f0 * (8.5 + 147.0 * k) + (r0 ? 5.0 + ((r0 <= 256 ? 43.0 : 57.0) + 0.17 * r0) * k : 0.0) +
+                       rounds0 * (scalar ? (epi == EPI_GATE_RES ? 54.0 : 16.0) : edge ? 6.0 : 0.0);
+    const double two = 8.0 + f1 * (12.7 + 115.0 * k) + (r1 ? 11.7 + (59.0 + 0.18 * r1) * k : 0.0) +
+                       0.0024 * N * k + (scalar ? 9.0 * rounds1 : 0.0);
+    return two < 0.97 * one;
 }
 
 constexpr size_t G256_MAX_BYTES = (size_t)1 << 30;  // fp16 fragments a product may ask for

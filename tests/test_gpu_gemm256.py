@@ -3,10 +3,15 @@ fragments; k_gemm on the weights in place, which a call takes under capture)
 give the same bits: an eager call against replays of the same call captured.
 k_gemm itself is compared with the oracle in the tests of the GEMM path.
 
+Which of them ran shows in the free memory: the decoded weights are the only
+thing an eager prepared product of this size allocates.
+
 Shapes: the edges of the 256 x 256 tile in tokens and rows, output widths that
 take the 16-byte stores, the scalar ones and both with a misaligned y, the
 shortest K (one super-block: eight stages, two turns of the four-stage ring) and
-one that is no multiple of the four super-blocks k_wfrag's workgroup decodes.
+ones that are no multiple of the four super-blocks k_wfrag's workgroup decodes;
+activations of 2^-20 to 2^20 by the row, with outliers, a row of zeros, an infinity
+and a NaN; short rows of whole tiles, which k_gemm takes.
 """
 import ctypes
 
@@ -24,11 +29,44 @@ def _weights(F, rng, name, N, K):
     return H.random_blocks(rng, name, N, K, scale_lo=-12, scale_hi=-8)
 
 
-def _both(F, call, dy, y0):
-    """The call run eagerly, then its captured form replayed twice (device-side fill between)."""
+def _free_bytes(F):
+    """Free device memory, through the library's own HIP runtime."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert F.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def _fragment_bytes(K, N, epi):
+    return ((N // 2 + 127) // 128 if epi == 2 else (N + 255) // 256) * 256 * K * 2
+
+
+def _same(a, b):
+    nan = np.isnan(a)
+    return np.array_equal(nan, np.isnan(b)) and np.array_equal(a[~nan].view(np.uint32), b[~nan].view(np.uint32))
+
+
+@pytest.fixture
+def fresh(gpu):
+    """The library without any workspace yet (shutdown frees it): a product that
+    decodes its weights then takes their bytes from the free memory."""
+    gpu.synchronize()
+    gpu.shutdown()
+    gpu.init(0)
+    yield gpu
+    gpu.synchronize()
+
+
+def _both(F, call, dy, y0, decoded):
+    """The call run eagerly, then its captured form replayed twice (device-side
+    fill between); decoded: the bytes of decoded weights the eager call must take,
+    or 0 if it must take none."""
     dy.upload(y0)
+    F.synchronize()
+    before = _free_bytes(F)
     call()
     F.synchronize()
+    taken = before - _free_bytes(F)
+    assert taken >= decoded if decoded else taken <= 0, (taken, decoded)
     eager = dy.download(np.float32, y0.shape)
     g = F.capture(call)
     try:
@@ -36,46 +74,54 @@ def _both(F, call, dy, y0):
             dy.upload(y0)
             g.launch()
             F.synchronize()
-            assert np.array_equal(eager.view(np.uint32), dy.download(np.float32, y0.shape).view(np.uint32)), rep
+            assert _same(eager, dy.download(np.float32, y0.shape)), rep
     finally:
         g.close()
     return eager
 
 
-# tokens x rows chosen so that the tile counts take k_gemm256 by its rule; the
-# last case is below it (both calls then run k_gemm)
+# (type, tokens, K, rows, epilogue, byte offset of y, whether the rule takes k_gemm256)
 CASES = [
-    ("Q4_K", 4097, 256, 5001, 0, 0), ("Q4_K", 4097, 512, 5004, 0, 0), ("Q4_K", 4100, 768, 5120, 0, 4),
-    ("Q4_K", 4095, 1280, 4993, 1, 0), ("Q4_K", 4096, 256, 5248, 1, 4), ("Q4_K", 4351, 512, 5248, 2, 0),
-    ("Q4_K", 4097, 256, 5376, 2, 4), ("Q5_K", 4097, 512, 5001, 0, 0), ("Q5_K", 4352, 1280, 4992, 0, 0),
-    ("Q6_K", 4097, 512, 5001, 0, 0), ("Q6_K", 4352, 1280, 4992, 0, 0), ("Q4_K", 1025, 256, 1001, 0, 0),
+    ("Q4_K", 4097, 256, 5001, 0, 0, 1), ("Q4_K", 16384, 1792, 1004, 0, 0, 1), ("Q4_K", 16384, 1792, 1004, 0, 4, 1),
+    ("Q4_K", 2561, 5120, 5120, 0, 0, 1), ("Q4_K", 4095, 1280, 4993, 1, 0, 1), ("Q4_K", 16384, 1792, 1004, 1, 0, 1),
+    ("Q4_K", 16383, 1792, 1004, 1, 4, 1), ("Q4_K", 3016, 2816, 10752, 2, 0, 1), ("Q4_K", 4097, 3840, 10752, 2, 4, 1),
+    ("Q5_K", 4097, 512, 5001, 0, 0, 1), ("Q5_K", 16384, 1280, 1000, 0, 0, 1), ("Q6_K", 4097, 512, 5001, 0, 0, 1),
+    ("Q6_K", 16384, 1280, 1000, 0, 0, 1), ("Q4_K", 1025, 256, 1001, 0, 0, 0), ("Q4_K", 4096, 512, 5120, 0, 0, 0),
 ]
 
 
-@pytest.mark.parametrize("name,M,K,N,epi,off", CASES)
-def test_eager_equals_captured(gpu, name, M, K, N, epi, off):
-    F = gpu
+@pytest.mark.parametrize("name,M,K,N,epi,off,takes", CASES)
+def test_eager_equals_captured(fresh, name, M, K, N, epi, off, takes):
+    F = fresh
     print("gemm256 %s M=%d K=%d N=%d epi=%d offset %d" % (name, M, K, N, epi, off), flush=True)
     rng = np.random.default_rng(M + N)
     qt = H.QTYPES[name][0]
-    x = rng.standard_normal((M, K)).astype(np.float32)
+    x = rng.standard_normal((M, K), dtype=np.float32) * np.exp2(rng.integers(-20, 21, (M, 1))).astype(np.float32)
+    x[rng.random((M, K)) < 0.01] *= 64
+    x[5] = 0
+    x[M - 1, K // 2] = np.inf
+    x[M // 2, 0] = np.nan
     W = N // 2 if epi == 2 else N
     dw, dx = F.DeviceBuffer.from_array(_weights(F, rng, name, N, K)), F.DeviceBuffer.from_array(x)
     db = F.DeviceBuffer.from_array(rng.standard_normal(N).astype(np.float32))
+    prep = F.DeviceBuffer(F.prepared_bytes(M, K))
+    F.prepare_x_dev(dx, M, K, prep)
     extra = off // 4
-    y0 = rng.standard_normal(M * W + extra).astype(np.float32)  # the gate residual adds to it
+    y0 = rng.standard_normal(M * W + extra, dtype=np.float32)  # the gate residual adds to it
     dy = F.DeviceBuffer(y0.nbytes)
-    dg = F.DeviceBuffer.from_array(rng.standard_normal(M * W + extra).astype(np.float32)) if epi == 1 else None
+    dg = F.DeviceBuffer.from_array(rng.standard_normal(M * W + extra, dtype=np.float32)) if epi == 1 else None
 
     def call():
         if epi == 0:
-            F.matmul_dev(dw, K, N, dx, dy.ptr + off, M, db, qtype=qt)
+            F.matmul_prepared_dev(dw, K, N, prep, dy.ptr + off, M, db, qtype=qt)
         else:
-            F.matmul_epi_dev(dw, K, N, dx, M, epi, dy.ptr + off, dg.ptr + off if dg else None, db)
+            F.matmul_prepared_epi_dev(dw, K, N, prep, M, epi, dy.ptr + off, dg.ptr + off if dg else None, db)
 
-    y = _both(F, call, dy, y0)
-    assert np.isfinite(y).all() and np.array_equal(y[:extra], y0[:extra])
-    for b in (dw, dx, db, dy, dg):
+    y = _both(F, call, dy, y0, _fragment_bytes(K, N, epi) if takes else 0)
+    ok = np.isfinite(x).all(1)
+    rows = y[extra:].reshape(M, W)
+    assert np.isfinite(rows[ok]).all() and not np.isfinite(rows[~ok]).any() and np.array_equal(y[:extra], y0[:extra])
+    for b in (dw, dx, db, prep, dy, dg):
         if b is not None:
             b.close()
 
@@ -84,7 +130,7 @@ def test_streams_share_the_decoded_weights_safely(gpu):
     """Prepared products of different weights on two streams, back to back
     without a wait between: each result is the one its call gives alone."""
     F = gpu
-    M, K, N = 4096, 512, 5120
+    M, K, N = 4096, 512, 5001
     print("gemm256 two streams M=%d K=%d N=%d" % (M, K, N), flush=True)
     rng = np.random.default_rng(5)
     x = rng.standard_normal((M, K)).astype(np.float32)
