@@ -577,16 +577,19 @@ __global__ __launch_bounds__(64 * NW, 2) void k_attn_fwd(const _Float16 *__restr
 // ---------------------------------------------------------------------------
 
 // scores[h][i][j] = (sum_d qp[h][i][d] * kp[h][j][d], in order) * scale
-// 64 x 64 tiles from LDS, 4 x 4 of them to a thread (rows and columns 16
+// TS x TS tiles from LDS, TS/16 x TS/16 of them to a thread (rows and columns 16
 // apart: the eight lanes of a 16-byte LDS read then start on different banks).
-// Bound by the separate products and sums; 245 tiles x 56 heads: 194 -> 36 us
-// (before: every dot product read its whole key row from memory).
-template <int HD>
+// TS = 64 is bound by the separate products and sums; 245 tiles x 56 heads: 194 ->
+// 36 us (before: every dot product read its whole key row from memory).  With few
+// tiles it takes as long as one such tile, 12 us: 16 x 16 ones then (1 tile x 16
+// heads 3.3 us, 100 x 16 5.7 against 13.4; 245 x 56 38.6 against 35.8).
+template <int HD, int TS>
 __global__ __launch_bounds__(256) void k_vsa_scores(const float *__restrict__ qp, const float *__restrict__ kp,
                                                     int T, float scale, float *__restrict__ sc) {
-    __shared__ __align__(16) float sq[64][HD + 4], sk[64][HD + 4];
-    const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64, h = blockIdx.z, t = threadIdx.x;
-    for (int c = t; c < 64 * HD / 4; c += 256) {
+    constexpr int X = TS / 16;
+    __shared__ __align__(16) float sq[TS][HD + 4], sk[TS][HD + 4];
+    const int i0 = blockIdx.y * TS, j0 = blockIdx.x * TS, h = blockIdx.z, t = threadIdx.x;
+    for (int c = t; c < TS * HD / 4; c += 256) {
         const int r = c / (HD / 4), d = 4 * (c % (HD / 4));
         const int i = i0 + r < T ? i0 + r : T - 1, j = j0 + r < T ? j0 + r : T - 1;
         *(f32x4 *)&sq[r][d] = *(const f32x4 *)(qp + ((size_t)h * T + i) * HD + d);
@@ -594,26 +597,26 @@ __global__ __launch_bounds__(256) void k_vsa_scores(const float *__restrict__ qp
     }
     __syncthreads();
     const int ti = t >> 4, tj = t & 15;
-    float dot[4][4] = {};
+    float dot[X][X] = {};
 #pragma unroll 4
     for (int d = 0; d < HD; d += 4) {
-        f32x4 a[4], b[4];
+        f32x4 a[X], b[X];
 #pragma unroll
-        for (int x = 0; x < 4; x++) {
+        for (int x = 0; x < X; x++) {
             a[x] = *(const f32x4 *)&sq[ti + 16 * x][d];
             b[x] = *(const f32x4 *)&sk[tj + 16 * x][d];
         }
 #pragma unroll
         for (int e = 0; e < 4; e++)
 #pragma unroll
-            for (int x = 0; x < 4; x++)
+            for (int x = 0; x < X; x++)
 #pragma unroll
-                for (int y = 0; y < 4; y++) dot[x][y] = dot[x][y] + a[x][e] * b[y][e];
+                for (int y = 0; y < X; y++) dot[x][y] = dot[x][y] + a[x][e] * b[y][e];
     }
 #pragma unroll
-    for (int x = 0; x < 4; x++)
+    for (int x = 0; x < X; x++)
 #pragma unroll
-        for (int y = 0; y < 4; y++) {
+        for (int y = 0; y < X; y++) {
             const int i = i0 + ti + 16 * x, j = j0 + tj + 16 * y;
             if (i < T && j < T) sc[((size_t)h * T + i) * T + j] = dot[x][y] * scale;
         }
@@ -700,7 +703,11 @@ __global__ __launch_bounds__(128) void k_vsa_lists(const float *__restrict__ sc,
 // Gated coarse branch: per (query tile i, head h) a softmax over all tile
 // scores mixes the pooled v: coarse[h][i][d] = sum_j expf(s_j - max) / sum * vp[h][j][d].
 // A workgroup takes RB query tiles, so that each pooled v is read once for all of
-// them: 245 tiles x 56 heads 84 -> 47 us.
+// them; bound by the latency of those reads, hence the unrolling.  245 tiles x 56
+// heads: one query tile (4 reads ahead) 84, eight 45, eight with 8 reads ahead 38
+// us.  Few workgroups or more than 32 KB of weights are better off with one query
+// tile and 16 reads ahead: 245 x 1 10.3 us (eight 29.5), 245 x 16 23.4 (31.0), 4096 x 4
+// 1326 (two 2931).
 template <int HD, int RB>
 __global__ __launch_bounds__(HD) void k_vsa_coarse(const float *__restrict__ sc, const float *__restrict__ vp,
                                                    int T, float *__restrict__ coarse) {
@@ -754,7 +761,8 @@ __global__ __launch_bounds__(HD) void k_vsa_coarse(const float *__restrict__ sc,
         for (int x = 0; x < RB; x++) wsh[j * RB + x] = wsh[j * RB + x] * sum[x];
     __syncthreads();
     const float *vcol = vp + (size_t)h * T * HD + d;
-#pragma unroll 4
+    constexpr int AHEAD = RB == 1 ? 16 : 8;
+#pragma unroll AHEAD
     for (int j = 0; j < T; j++) {
         const float v = vcol[(size_t)j * HD];
 #pragma unroll
@@ -865,14 +873,19 @@ hipError_t vsa_launch(const float *q, const float *k, const float *v, int64_t ld
     hipLaunchKernelGGL((cosb && rot % 8 ? k_attn_prep<HD, true> : k_attn_prep<HD, false>),
                        dim3(n_pad / ATT_PREP_T, (heads + G - 1) / G), dim3(512), 0, st, q, k, v, ld, ldv, ATT_KT * T,
                        heads, G, gather, qn_w, kn_w, eps, cosb, sinb, rot, qscale, n_pad, w.Qp, w.Kp, w.Vt, pl);
-    const int t64 = (T + 63) / 64;
-    hipLaunchKernelGGL((k_vsa_scores<HD>), dim3(t64, t64, heads), dim3(256), 0, st, w.qp, w.kp, T, scale, w.sc);
+    // 16 x 16 score tiles while 64 x 64 ones would leave CUs without any
+    const int t64 = (T + 63) / 64, t16 = (T + 15) / 16;
+    if ((int64_t)t64 * t64 * heads < 256)
+        hipLaunchKernelGGL((k_vsa_scores<HD, 16>), dim3(t16, t16, heads), dim3(256), 0, st, w.qp, w.kp, T, scale, w.sc);
+    else
+        hipLaunchKernelGGL((k_vsa_scores<HD, 64>), dim3(t64, t64, heads), dim3(256), 0, st, w.qp, w.kp, T, scale, w.sc);
     hipLaunchKernelGGL((T <= 256 ? k_vsa_lists<4> : T <= 1024 ? k_vsa_lists<16> : k_vsa_lists<64>), dim3(nqb, heads),
                        dim3(128), 0, st, w.sc, T, P, kv, all, nqb, w.lists, w.list_len);
     if (gate) {
-        // eight query tiles to a workgroup while their weights take at most 32 KB of LDS
-        const int rb = T <= 1024 ? 8 : 2;
-        hipLaunchKernelGGL((rb == 8 ? k_vsa_coarse<HD, 8> : k_vsa_coarse<HD, 2>), dim3((T + rb - 1) / rb, heads),
+        // eight query tiles to a workgroup while that leaves three of them to a CU and their weights take at
+        // most 32 KB of LDS
+        const int rb = T <= 1024 && (int64_t)((T + 7) / 8) * heads >= 768 ? 8 : 1;
+        hipLaunchKernelGGL((rb == 8 ? k_vsa_coarse<HD, 8> : k_vsa_coarse<HD, 1>), dim3((T + rb - 1) / rb, heads),
                            dim3(HD), (size_t)T * rb * sizeof(float), st, w.sc, w.vp, T, w.coarse);
     }
     Sparse sp{w.lists, w.list_len, cnt, gather, gate ? w.coarse : nullptr, gate, T};
