@@ -16,6 +16,7 @@
 
 #include "fh3/fh3.h"
 #include "fh3/fh3_hip.h"
+#include "fh3_fragments.h"
 #include "fh3_kernels.h"
 #include "fh3_hip_internal.h"
 
@@ -26,6 +27,49 @@ struct DevBuf {
     size_t cap = 0;
 };
 
+bool is_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// The runtime calls of the weight fragments; a failed one leaves no error behind.
+struct FragRt {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    // allocate and free without disturbing a capture of this or another thread
+    struct Relaxed {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+        ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    };
+    static bool ok(hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
+    }
+    bool capturing(Stream st) const { return is_capturing(st); }
+    void *alloc(size_t bytes) const {
+        Relaxed r;
+        void *p = nullptr;
+        return ok(hipMalloc(&p, bytes)) ? p : nullptr;
+    }
+    void free(void *p) const {
+        Relaxed r;
+        ok(hipFree(p));
+    }
+    bool create(Event &e) const {
+        if (ok(hipEventCreateWithFlags(&e, hipEventDisableTiming))) return true;
+        e = nullptr;
+        return false;
+    }
+    void destroy(Event e) const { ok(hipEventDestroy(e)); }
+    bool wait(Stream st, Event e) const { return ok(hipStreamWaitEvent(st, e, 0)); }
+    bool record(Event e, Stream st) const { return ok(hipEventRecord(e, st)); }
+    void sync(Event e) const {
+        Relaxed r;
+        ok(hipEventSynchronize(e));
+    }
+};
+
 struct State {
     bool init = false;
     int device = -1;
@@ -33,8 +77,7 @@ struct State {
     DevBuf ws;                      // x16 fragments + per-row scales
     DevBuf ws2;                     // x16 made from a prepared fp32 copy (other weight types)
     DevBuf w16;                     // fp16 rows of a weight of another type
-    DevBuf wfrag;                   // fp16 fragments of a large product's weights (wfrag_take)
-    hipEvent_t wfrag_used = nullptr;  // after the last product that read wfrag
+    WeightFragments<FragRt> wfrag;  // fp16 fragments of a large product's weights
     DevBuf part;                    // split-K partial sums of the middle-M kernel
     DevBuf attn;                    // fp16 attention operands (Qp, Kp, Vt)
     DevBuf vsa_ws;                  // VSA operands, tile statistics, scores and tile lists
@@ -95,11 +138,6 @@ int ensure_init() {
     return fh3_hip_init(env ? atoi(env) : 0);
 }
 
-bool capturing(hipStream_t st) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
-}
-
 // Give up b's allocation: freed once the device is idle (enqueued kernels may
 // still read it), or kept until fh3_hip_graph_destroy has destroyed the last
 // graph when captured graphs exist (their kernels hold its address).
@@ -120,7 +158,7 @@ int release(DevBuf &b) {
 // Grow-only device buffer.  A grow allocates, so it is refused while `st` is
 // being captured into a graph: the call must have run once eagerly first.
 int grow(DevBuf &b, size_t need, hipStream_t st) {
-    const bool cap = capturing(st);
+    const bool cap = is_capturing(st);
     // a graph the library does not own may now hold this buffer's address
     if (cap && !t_own_capture) g.foreign_capture = true;
     if (b.cap >= need) return FH3_OK;
@@ -133,49 +171,6 @@ int grow(DevBuf &b, size_t need, hipStream_t st) {
     FH3_HIPCALL(hipMalloc(&b.p, need));
     b.cap = need;
     return FH3_OK;
-}
-
-// The large products' weight fragments, for one product on `st` (g.mu held;
-// wfrag_release after its launches).  One buffer serves every stream: each user
-// waits on the device for the one before it, so products on different
-// streams stay safe, as they were when k_gemm needed no such memory.  NULL -- the
-// product then reads its weights in place (k_gemm, the same bits) -- when the
-// stream is being captured (a graph must not hold the shared buffer or wait
-// for events outside it) or the memory is not to be had.
-void *wfrag_take(size_t bytes, hipStream_t st) {
-    if (capturing(st)) return nullptr;
-    if (!g.wfrag_used && hipEventCreateWithFlags(&g.wfrag_used, hipEventDisableTiming) != hipSuccess) {
-        g.wfrag_used = nullptr;
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (g.wfrag.cap < bytes) {
-        // allocate and free without disturbing another thread's capture
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-        if (g.wfrag.p) {
-            (void)hipEventSynchronize(g.wfrag_used);
-            (void)hipFree(g.wfrag.p);
-        }
-        g.wfrag = DevBuf();
-        const hipError_t e = hipMalloc(&g.wfrag.p, bytes);
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-        if (e != hipSuccess) {
-            g.wfrag.p = nullptr;
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        g.wfrag.cap = bytes;
-    } else if (hipStreamWaitEvent(st, g.wfrag_used, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return g.wfrag.p;
-}
-
-hipError_t wfrag_release(hipStream_t st) {
-    const hipError_t e = hipEventRecord(g.wfrag_used, st);
-    return e == hipSuccess ? e : hipStreamSynchronize(st);
 }
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
@@ -339,15 +334,14 @@ extern "C" void fh3_hip_shutdown(void) {
     std::lock_guard<std::recursive_mutex> lk(g.mu);
     if (!g.init) return;
     (void)hipDeviceSynchronize();
-    DevBuf *bufs[] = {&g.ws, &g.ws2, &g.w16, &g.wfrag, &g.part, &g.attn, &g.vsa_ws, &g.vsa_geo,
+    DevBuf *bufs[] = {&g.ws, &g.ws2, &g.w16, &g.part, &g.attn, &g.vsa_ws, &g.vsa_geo,
                       &g.st_w, &g.st_x, &g.st_y, &g.st_b};
     for (DevBuf *b : bufs) {
         if (b->p) (void)hipFree(b->p);
         b->p = nullptr;
         b->cap = 0;
     }
-    if (g.wfrag_used) (void)hipEventDestroy(g.wfrag_used);
-    g.wfrag_used = nullptr;
+    g.wfrag.clear();
     for (auto &r : g.regs) (void)hipFree(r.dev);
     g.regs.clear();
     for (void *p : g.retired) (void)hipFree(p);
@@ -630,12 +624,12 @@ static int product_wfrag(const Fh3W *w, const void *x16, const float *xs_inv, in
     *done = false;
     const int K = (int)w->in, N = (int)w->out;
     const size_t wb = fh3k_gemm256_bytes(w->type, N, K, n_tok, epi);
-    void *wf = wb ? wfrag_take(wb, st) : nullptr;
+    void *wf = wb ? g.wfrag.take(wb, st) : nullptr;
     if (!wf) return FH3_OK;
     *done = true;
     const hipError_t e = fh3k_gemm256(w->type, w->data, (int64_t)fh3_row_bytes(w->type, w->in), N, K, x16, xs_inv, bias,
                                       d_y, n_tok, epi, aux, wf, st);
-    const hipError_t r = wfrag_release(st);
+    const hipError_t r = g.wfrag.give(st) ? hipSuccess : hipStreamSynchronize(st);
     FH3_HIPCALL(e);
     FH3_HIPCALL(r);
     return FH3_OK;
@@ -1099,7 +1093,7 @@ static int vsa_plan(const Fh3Seq *sq, int tile, hipStream_t st, const char *fn) 
     const int key[8] = {sq->seq_len, sq->num_text, sq->num_audio, sq->num_video, sq->grid_t, sq->grid_h, sq->grid_w,
                         tile};
     if (memcmp(key, g.vsa_key, sizeof key) == 0) return FH3_OK;
-    if (capturing(st))
+    if (is_capturing(st))
         return set_err(FH3_E_INVALID, "%s: a new sequence shape during graph capture; run the call once eagerly "
                                       "before capturing it", fn);
     std::vector<int> tok, off;
