@@ -3870,10 +3870,11 @@ static hipError_t launch_gemm256(const void *W, int64_t row_bytes, int N, int K,
 // overlaps neither), the launches, the decode, and the scalar stores of rows
 // that are no multiple of 4 floats and of k_gemm's last columns.  Fitted to 673 shapes
 // (K 256-25600, N 1000-28672, 1024-32768 tokens, every type and epilogue) with both
-// forms timed: 7 / 5 % rms.  What they choose is 10.6 % faster than k_gemm alone
-// (geometric mean; 11.3 the better form each time), at worst 6 % slower at K >=
-// 1024; with times that only scaled with K (8.4 %) 96 of the shapes had become
-// slower: 2048 x 1024 -> 5120 31.6 -> 40.7 us, now 31.6; 2048 x 256 -> 5120 15.7 -> 24.6.
+// forms timed: 7 / 5 % rms (2 of the 10 us are the margin by which k_gemm256
+// has to win).  What they choose is 10.7 % faster than k_gemm alone (geometric
+// mean; 11.3 the better form each time), at worst 6 % slower; with times that only
+// scaled with K (8.4 %) 96 of the shapes had become slower: 2048 x 1024 -> 5120
+// 31.6 -> 40.7 us, now 31.6; 2048 x 256 -> 5120 15.7 -> 24.6.
 // Only where k_gemm does not split K: the two then give the same bits, which one
 // a call takes cannot be told from its result.
 static bool gemm256_wins(int N, int K, int M, int epi) {
@@ -3889,9 +3890,9 @@ static bool gemm256_wins(int N, int K, int M, int epi) {
     const bool scalar = (sw ? N / 2 : N) % 4 != 0, edge = !sw && !scalar && N % GEMM_BN;
     const double one = 7.0 + f0 * (8.5 + 147.0 * k) + (r0 ? 5.0 + ((r0 <= 256 ? 43.0 : 57.0) + 0.17 * r0) * k : 0.0) +
                        rounds0 * (scalar ? (epi == EPI_GATE_RES ? 54.0 : 16.0) : edge ? 6.0 : 0.0);
-    const double two = 8.0 + f1 * (12.7 + 115.0 * k) + (r1 ? 11.7 + (59.0 + 0.18 * r1) * k : 0.0) +
+    const double two = 10.0 + f1 * (12.7 + 115.0 * k) + (r1 ? 11.7 + (59.0 + 0.18 * r1) * k : 0.0) +
                        0.0024 * N * k + (scalar ? 9.0 * rounds1 : 0.0);
-    return two < 0.97 * one;
+    return two < one;
 }
 
 constexpr size_t G256_MAX_BYTES = (size_t)1 << 30;  // fp16 fragments a product may ask for
