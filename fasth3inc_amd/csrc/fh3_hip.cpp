@@ -64,6 +64,10 @@ struct FragRt {
     void destroy(Event e) const { ok(hipEventDestroy(e)); }
     bool wait(Stream st, Event e) const { return ok(hipStreamWaitEvent(st, e, 0)); }
     bool record(Event e, Stream st) const { return ok(hipEventRecord(e, st)); }
+    bool done(Event e) const {
+        Relaxed r;
+        return ok(hipEventQuery(e));
+    }
     void sync(Event e) const {
         Relaxed r;
         ok(hipEventSynchronize(e));

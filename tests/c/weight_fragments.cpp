@@ -38,6 +38,7 @@ struct Fake {
     void destroy(int) {}
     bool wait(int, int e) { return b.waits.push_back(e), true; }
     bool record(int e, int) { return b.busy.insert(e), true; }
+    bool done(int e) { return !b.busy.count(e); }
     void sync(int e) { b.busy.erase(e); }
 };
 
@@ -71,7 +72,34 @@ static int capture() {
     return 0;
 }
 
+// Streams 1, 2 and 3 at work at once: two buffers, no stream waits for another
+// and no buffer is used under one that is still at work.
+static int streams() {
+    b = Books();
+    WeightFragments<Fake> w;
+    void *p = w.take(100, 1);
+    CHECK(p && w.give(1));
+    void *q = w.take(100, 2);
+    CHECK(q && q != p && w.give(2) && b.waits.empty());
+    CHECK(!w.take(100, 3) && !w.take(10, 3) && b.waits.empty() && b.allocs == 2);
+    CHECK(w.take(100, 1) == p && w.give(1));  // behind its own stream's work
+    CHECK(b.waits == std::vector<int>{1});
+    CHECK(w.take(100, 2) == q && w.give(2));
+    b.busy.erase(1);  // stream 1's work ends: a third stream takes its buffer
+    CHECK(w.take(100, 3) == p && w.give(3));
+    CHECK(!w.take(100, 1) && b.allocs == 2);
+    void *r = w.take(200, 2);  // a stream's own buffer grows behind its work, the others stay
+    CHECK(r && w.give(2) && b.live.count(p) && !b.live.count(q) && b.held == 300);
+    b.busy.clear();
+    CHECK(w.take(150, 3) == r && w.give(3));  // the idle one is large enough: no growth
+    CHECK(b.allocs == 3);
+    w.clear();
+    CHECK(b.held == 0);
+    return 0;
+}
+
 int main() {
+    if (int r = streams()) return r;
     if (int r = growth()) return r;
     if (int r = capture()) return r;
     return 0;

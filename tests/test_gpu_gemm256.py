@@ -156,3 +156,54 @@ def test_streams_share_the_decoded_weights_safely(gpu):
         assert np.array_equal(dy.download(np.uint32, (M, N)), w)
     for s in streams:
         assert F.lib().hipStreamDestroy(s) == 0
+
+
+@pytest.fixture
+def streams(fresh):
+    """Three streams of the library's own HIP runtime; 1 = hipStreamNonBlocking."""
+    made = [ctypes.c_void_p() for _ in range(3)]
+    for s in made:
+        assert fresh.lib().hipStreamCreateWithFlags(ctypes.byref(s), ctypes.c_uint(1)) == 0
+    yield made
+    fresh.synchronize()
+    for s in made:
+        assert fresh.lib().hipStreamDestroy(s) == 0
+
+
+def test_streams_side_by_side(fresh, streams):
+    """Prepared products of different weights and sizes on three streams, back to
+    back without a wait between (two have decoded weights of their own, which
+    grow while the others' products are at work, the third reads in place
+    meanwhile): each result is the one its call gives alone."""
+    F = fresh
+    M = 4096
+    shapes = [(512, 5001), (768, 5001), (1280, 5001)]
+    print("gemm256 three streams M=%d" % M, flush=True)
+    rng = np.random.default_rng(5)
+    work = []
+    for K, N in shapes:
+        dx, prep = F.DeviceBuffer.from_array(rng.standard_normal((M, K), dtype=np.float32)), F.DeviceBuffer(F.prepared_bytes(M, K))
+        F.prepare_x_dev(dx, M, K, prep)
+        dw = F.DeviceBuffer.from_array(F.synth_q4k_weights(K, 1, N, K, 0.05, 0.0))
+        work.append((K, N, dw, prep))
+    F.synchronize()
+    want = []
+    for K, N, dw, prep in work:  # captured: read in place, nothing decoded before the streams run
+        dy = F.DeviceBuffer(M * N * 4)
+        g = F.capture(lambda: F.matmul_prepared_dev(dw, K, N, prep, dy, M))
+        g.launch()
+        F.synchronize()
+        want.append(dy.download(np.uint32, (M, N)))
+        g.close()
+    before = _free_bytes(F)
+    dys = [[F.DeviceBuffer(M * N * 4) for K, N in shapes] for _ in streams]
+    ys = before - _free_bytes(F)
+    for k in range(6):  # every stream runs every shape, small to large
+        for i, s in enumerate(streams):
+            K, N, dw, prep = work[(k // 2) % 3]
+            F.matmul_prepared_dev(dw, K, N, prep, dys[i][(k // 2) % 3], M, stream_ptr=s)
+    F.synchronize()
+    assert before - _free_bytes(F) - ys >= _fragment_bytes(1280, 5001, 0), "no product decoded its weights"
+    for per_stream in dys:
+        for dy, w in zip(per_stream, want):
+            assert np.array_equal(dy.download(np.uint32, w.shape), w)
