@@ -4,6 +4,7 @@
 // Rt stands for the HIP runtime, so that the rules below also run without a GPU:
 //   Rt::Stream, Rt::Event (value types; Event{} is none)
 //   bool capturing(Stream)          void *alloc(size_t)         void free(void *)
+//   size_t available()  (bytes of device memory that are free)
 //   bool create(Event &)            bool wait(Stream, Event)    bool record(Event, Stream)
 //   bool done(Event)                void sync(Event)            void destroy(Event)
 #ifndef FH3_FRAGMENTS_H
@@ -44,6 +45,19 @@ public:
     // The product's launches are on `st`; false: the caller must wait for them.
     bool give(Stream st) { return rt.record(taken->used, st); }
 
+    // Every buffer back to the device, once its work has ended; false: there was none.
+    bool trim() {
+        bool any = false;
+        for (Slot &s : slots)
+            if (s.p) {
+                rt.sync(s.used);
+                rt.free(s.p);
+                s.p = nullptr, s.cap = 0;
+                any = true;
+            }
+        return any;
+    }
+
     void clear() {
         for (Slot &s : slots) {
             if (s.p) rt.free(s.p);
@@ -80,7 +94,10 @@ private:
     }
 
     // The old buffer stays until the new one is there, and for good if it is refused.
+    // At most an eighth of the free memory is taken: k_gemm needs none, and what is
+    // left is the caller's.
     bool grow(Slot &s, size_t bytes) {
+        if (bytes > rt.available() / 8) return false;
         if (s.used == Event{} && !rt.create(s.used)) return false;
         void *q = rt.alloc(bytes);
         if (!q) return false;

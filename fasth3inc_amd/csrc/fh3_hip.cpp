@@ -47,6 +47,11 @@ struct FragRt {
         return e == hipSuccess;
     }
     bool capturing(Stream st) const { return is_capturing(st); }
+    size_t available() const {
+        Relaxed r;
+        size_t free = 0, total = 0;
+        return ok(hipMemGetInfo(&free, &total)) ? free : 0;
+    }
     void *alloc(size_t bytes) const {
         Relaxed r;
         void *p = nullptr;
@@ -142,6 +147,16 @@ int ensure_init() {
     return fh3_hip_init(env ? atoi(env) : 0);
 }
 
+// hipMalloc; where the memory is not there, once more without the decoded weights' buffers.
+hipError_t dev_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    std::lock_guard<std::recursive_mutex> lk(g.mu);
+    if (!g.wfrag.trim()) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
 // Give up b's allocation: freed once the device is idle (enqueued kernels may
 // still read it), or kept until fh3_hip_graph_destroy has destroyed the last
 // graph when captured graphs exist (their kernels hold its address).
@@ -172,7 +187,7 @@ int grow(DevBuf &b, size_t need, hipStream_t st) {
                        "run the call once eagerly before capturing it", need);
     int rc = release(b);
     if (rc != FH3_OK) return rc;
-    FH3_HIPCALL(hipMalloc(&b.p, need));
+    FH3_HIPCALL(dev_malloc(&b.p, need));
     b.cap = need;
     return FH3_OK;
 }
@@ -368,7 +383,7 @@ extern "C" int fh3_hip_malloc(void **dptr, size_t bytes) {
     if (!dptr) return set_err(FH3_E_INVALID, "fh3_hip_malloc: NULL out pointer");
     int rc = ensure_init();
     if (rc != FH3_OK) return rc;
-    FH3_HIPCALL(hipMalloc(dptr, bytes ? bytes : 1));
+    FH3_HIPCALL(dev_malloc(dptr, bytes ? bytes : 1));
     return FH3_OK;
 }
 
@@ -1027,7 +1042,7 @@ extern "C" int fh3_hip_register_weights(const void *host, size_t bytes, const vo
             return set_err(FH3_E_INVALID, "%s: range overlaps a registered range", fn);
     }
     void *dev = nullptr;
-    FH3_HIPCALL(hipMalloc(&dev, bytes));
+    FH3_HIPCALL(dev_malloc(&dev, bytes));
     const hipError_t e = hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(dev);

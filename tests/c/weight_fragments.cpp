@@ -9,6 +9,7 @@
 
 struct Books {
     size_t limit = 1u << 30, held = 0;  // bytes the "device" has, and how many are allocated
+    size_t hidden = 0;                  // free bytes that no allocation gets
     int allocs = 0, events = 0;
     std::map<void *, size_t> live;
     std::set<int> busy;        // events whose work has not ended
@@ -21,9 +22,10 @@ struct Fake {
     using Stream = int;
     using Event = int;
     bool capturing(int st) { return b.captured.count(st) != 0; }
+    size_t available() { return b.limit - b.held; }
     void *alloc(size_t n) {
         b.allocs++;
-        if (b.held + n > b.limit) return nullptr;
+        if (b.held + n > b.limit - b.hidden) return nullptr;
         void *p = ::operator new(1);
         b.live[p] = n;
         b.held += n;
@@ -47,7 +49,7 @@ struct Fake {
 
 static int growth() {
     b = Books();
-    b.limit = 500;
+    b.limit = 5000, b.hidden = 4500;
     WeightFragments<Fake> w;
     void *p = w.take(100, 1);
     CHECK(p && w.give(1));
@@ -98,7 +100,22 @@ static int streams() {
     return 0;
 }
 
+// Memory that others need is left to them, and given back when they ask.
+static int memory() {
+    b = Books();
+    b.limit = 1000;
+    WeightFragments<Fake> w;
+    CHECK(!w.take(126, 1) && b.allocs == 0);  // more than an eighth of what is free
+    CHECK(w.take(125, 1) && w.give(1));
+    CHECK(!w.take(110, 2) && b.allocs == 1);  // of what is free now
+    CHECK(w.take(109, 2) && w.give(2) && b.held == 234);
+    CHECK(w.trim() && b.held == 0 && b.busy.empty() && !w.trim());
+    CHECK(w.take(125, 2) && w.give(2));
+    return 0;
+}
+
 int main() {
+    if (int r = memory()) return r;
     if (int r = streams()) return r;
     if (int r = growth()) return r;
     if (int r = capture()) return r;
