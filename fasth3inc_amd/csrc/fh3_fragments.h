@@ -5,6 +5,7 @@
 //   Rt::Stream, Rt::Event (value types; Event{} is none)
 //   bool capturing(Stream)          void *alloc(size_t)         void free(void *)
 //   size_t available()  (bytes of device memory that are free)
+//   Rt::On(int)  (the device is the calling thread's current one while it lives)
 //   bool create(Event &)            bool wait(Stream, Event)    bool record(Event, Stream)
 //   bool done(Event)                void sync(Event)            void destroy(Event)
 #ifndef FH3_FRAGMENTS_H
@@ -28,11 +29,13 @@ public:
     // not to be had.  No stream ever waits for another.
     // (2048 x 5120 -> 5120 on two streams: 124 us a product with one buffer whose
     // users waited for one another, 102 with k_gemm alone, 98 with two.)
-    void *take(size_t bytes, Stream st) {
+    // Memory and events are the library's device's, whichever the calling thread's is.
+    void *take(size_t bytes, Stream st, int device) {
         if (rt.capturing(st)) return nullptr;
         Slot *s = pick(bytes, st);
         if (!s) return nullptr;
         if (s->cap < bytes) {
+            typename Rt::On here(device);
             if (!grow(*s, bytes)) return nullptr;
         } else if (!rt.wait(st, s->used)) {  // for earlier work of this stream, or of one whose handle it has
             return nullptr;

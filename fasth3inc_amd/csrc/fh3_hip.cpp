@@ -36,6 +36,16 @@ bool is_capturing(hipStream_t st) {
 struct FragRt {
     using Stream = hipStream_t;
     using Event = hipEvent_t;
+    struct On {
+        int old = -1;
+        explicit On(int device) {
+            if (hipGetDevice(&old) != hipSuccess || old == device) old = -1;
+            else (void)hipSetDevice(device);
+        }
+        ~On() {
+            if (old >= 0) (void)hipSetDevice(old);
+        }
+    };
     // allocate and free without disturbing a capture of this or another thread
     struct Relaxed {
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -643,7 +653,7 @@ static int product_wfrag(const Fh3W *w, const void *x16, const float *xs_inv, in
     *done = false;
     const int K = (int)w->in, N = (int)w->out;
     const size_t wb = fh3k_gemm256_bytes(w->type, N, K, n_tok, epi);
-    void *wf = wb ? g.wfrag.take(wb, st) : nullptr;
+    void *wf = wb ? g.wfrag.take(wb, st, g.device) : nullptr;
     if (!wf) return FH3_OK;
     *done = true;
     const hipError_t e = fh3k_gemm256(w->type, w->data, (int64_t)fh3_row_bytes(w->type, w->in), N, K, x16, xs_inv, bias,
