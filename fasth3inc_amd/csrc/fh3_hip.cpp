@@ -816,6 +816,19 @@ static int check_epi(const Fh3W *w, int epi, const float *aux, const char *fn) {
     return FH3_OK;
 }
 
+// Whether a product of fp32 activations and F16 rows runs k_short16: no
+// preparation and no workspace.  Longer rows, whose operands do not fit one
+// workgroup, and forced paths take the general route.
+static bool takes_short16(const Fh3W *w, int n_tok) {
+    return w->type == FH3_QUANT_F16 && g.path == FH3_HIP_PATH_AUTO && w->in <= 128 &&
+           fh3k_short16_fits((int)w->in, (int)w->out, n_tok);
+}
+
+// Whether [a, a + an) and [b, b + bn) share bytes.
+static bool overlap(const void *a, size_t an, const void *b, size_t bn) {
+    return (uintptr_t)a < (uintptr_t)b + bn && (uintptr_t)b < (uintptr_t)a + an;
+}
+
 static int matmul_dev(const Fh3W *w, const float *d_x, float *d_y, int n_tok, const float *d_bias_or_null,
                       void *stream, int epi, const float *aux, const char *fn) {
     int rc = check_weights(w, fn);
@@ -828,10 +841,8 @@ static int matmul_dev(const Fh3W *w, const float *d_x, float *d_y, int n_tok, co
     rc = ensure_init();
     if (rc != FH3_OK) return rc;
     hipStream_t st = stream ? (hipStream_t)stream : g.stream;
-    if (w->type == FH3_QUANT_F16 && g.path == FH3_HIP_PATH_AUTO && w->in <= 128 &&
-        fh3k_short16_fits((int)w->in, (int)w->out, n_tok)) {
-        // no preparation and no workspace; longer rows, whose operands no longer fit one workgroup, take
-        // the general route below (at its shortest of 128: 10-191 us for 1-16384 tokens against 6-89 here)
+    // k_short16 reads x while it stores y, so a y that lies over x takes the general route, which has read x by then
+    if (takes_short16(w, n_tok) && !overlap(d_x, (size_t)n_tok * w->in * 4, d_y, (size_t)n_tok * w->out * 4)) {
         FH3_HIPCALL(fh3k_short16(w->data, (int)w->out, (int)w->in, d_x, d_bias_or_null, d_y, n_tok, st));
         return FH3_OK;
     }

@@ -43,3 +43,24 @@ def test_short_rows_same_bits(gpu, M, K, N, bias):
     ok = np.isfinite(x).all(1)
     ref = x[ok].astype(np.float64) @ w.astype(np.float64).T + (0 if b is None else b)
     assert H.rel_fro(out[0][:M][ok], ref) <= 1e-3  # one rounding of x to fp16 (2^-11) and fp32 sums
+
+
+@pytest.mark.parametrize("M,K,N,shift", [(300, 96, 96, 0), (257, 64, 128, 0), (1000, 128, 8, 0), (200, 96, 96, 4),
+                                         (300, 32, 64, -1000)])
+def test_output_over_the_activations(gpu, M, K, N, shift):
+    """y at x (shift floats further): the result is the one two buffers give."""
+    F = gpu
+    print("y over x M=%d K=%d N=%d shift %d" % (M, K, N, shift), flush=True)
+    rng = np.random.default_rng(M + N)
+    w = rng.standard_normal((N, K)).astype(np.float16)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    dw, dx, dy = F.DeviceBuffer.from_array(w), F.DeviceBuffer.from_array(x), F.DeviceBuffer(M * N * 4)
+    F.matmul_dev(dw, K, N, dx, dy, M, qtype=F.FH3_QUANT_F16)
+    both = F.DeviceBuffer((2000 + M * max(K, N)) * 4)
+    host = np.zeros(2000 + M * max(K, N), np.float32)
+    host[1000:1000 + M * K] = x.reshape(-1)
+    both.upload(host)
+    F.matmul_dev(dw, K, N, both.ptr + 4000, both.ptr + 4 * (1000 + shift), M, qtype=F.FH3_QUANT_F16)
+    F.synchronize()
+    got = both.download(np.float32, host.shape)[1000 + shift:1000 + shift + M * N]
+    assert np.array_equal(got.view(np.uint32), dy.download(np.uint32, (M * N,)))
