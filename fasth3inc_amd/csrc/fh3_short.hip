@@ -123,18 +123,24 @@ __global__ __launch_bounds__(256) void k_short16(const _Float16 *__restrict__ W1
     }
 }
 
+// Workgroups of M x N outputs, token tiles first; in 64 bits: M + 127 does not fit an int at the largest M.
+constexpr int64_t short_tiles(int64_t M, int64_t N) {
+    return (M + SHORT_M - 1) / SHORT_M * ((N + SHORT_N - 1) / SHORT_N);
+}
+static_assert(short_tiles(0x7FFFFFFF, 1) == 0x1000000 && short_tiles(0x7FFFFFFF, 0x7FFFFFFF) > 0x7FFFFFFF, "");
+
 }  // namespace
 
 extern "C" int fh3k_short16_fits(int K, int N, int M) {
-    const int64_t tiles = (int64_t)((M + SHORT_M - 1) / SHORT_M) * ((N + SHORT_N - 1) / SHORT_N);
-    return K >= 8 && K <= SHORT_K && K % 8 == 0 && tiles <= 0x7FFFFFFF;
+    return K >= 8 && K <= SHORT_K && K % 8 == 0 && N <= 0x7FFFFFFF - SHORT_N &&
+           short_tiles(M, N) <= 0xFFFFFF;  // a launch holds fewer than 2^32 threads
 }
 
 extern "C" hipError_t fh3k_short16(const void *W16, int N, int K, const float *x, const float *bias, float *y, int M,
                                    hipStream_t st) {
     if (!fh3k_short16_fits(K, N, M)) return hipErrorInvalidValue;
     const int n_tiles = (N + SHORT_N - 1) / SHORT_N;
-    hipLaunchKernelGGL(k_short16, dim3((unsigned)((M + SHORT_M - 1) / SHORT_M * n_tiles)), dim3(256), 0, st,
+    hipLaunchKernelGGL(k_short16, dim3((unsigned)short_tiles(M, N)), dim3(256), 0, st,
                        (const _Float16 *)W16, N, K, x, bias, y, M, n_tiles);
     return hipGetLastError();
 }
