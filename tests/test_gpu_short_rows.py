@@ -45,6 +45,30 @@ def test_short_rows_same_bits(gpu, M, K, N, bias):
     assert H.rel_fro(out[0][:M][ok], ref) <= 1e-3  # one rounding of x to fp16 (2^-11) and fp32 sums
 
 
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 33, 64, 65, 200])
+@pytest.mark.parametrize("K", [8, 24, 32, 96, 104, 128])
+def test_prepared_gives_the_same_bits(gpu, M, K):
+    """The two-stage form, which runs k_skinny16 up to 64 tokens and k_gemm16
+    above: rows of 2^-20 to 2^20, a row of zeros, an infinity, a NaN."""
+    F = gpu
+    N = 300
+    print("short rows, prepared and direct M=%d K=%d" % (M, K), flush=True)
+    rng = np.random.default_rng(M * 1000 + K)
+    w = (rng.standard_normal((N, K)) * np.exp2(rng.integers(-8, 9, (N, K)))).astype(np.float16)
+    x = (rng.standard_normal((M, K)) * np.exp2(rng.integers(-20, 21, (M, 1)))).astype(np.float32)
+    if M > 3:
+        x[1], x[2, K - 1], x[3, 0] = 0, np.inf, np.nan
+    dw, dx, db = (F.DeviceBuffer.from_array(a) for a in (w, x, rng.standard_normal(N).astype(np.float32)))
+    prep, dys = F.DeviceBuffer(F.prepared_bytes(M, K)), [F.DeviceBuffer(M * N * 4) for _ in range(2)]
+    F.matmul_dev(dw, K, N, dx, dys[0], M, db, qtype=F.FH3_QUANT_F16)
+    F.prepare_x_dev(dx, M, K, prep)
+    F.matmul_prepared_dev(dw, K, N, prep, dys[1], M, db, qtype=F.FH3_QUANT_F16)
+    F.synchronize()
+    a, b = (d.download(np.float32, (M, N)) for d in dys)
+    nan = np.isnan(a)
+    assert np.array_equal(nan, np.isnan(b)) and np.array_equal(a[~nan].view(np.uint32), b[~nan].view(np.uint32))
+
+
 @pytest.mark.parametrize("M,K,N,shift", [(300, 96, 96, 0), (257, 64, 128, 0), (1000, 128, 8, 0), (200, 96, 96, 4),
                                          (300, 32, 64, -1000)])
 def test_output_over_the_activations(gpu, M, K, N, shift):
