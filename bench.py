@@ -43,10 +43,10 @@ METRIC = "Q4_K GEMM TFLOP/s + GEMV weight GB/s (% roofline); DiT block linear ms
 # --reps 5` (and `gemm` for the GEMM figures), scaled by 2.0 and 1.0: a 256 MiB
 # device-to-device copy reads FETCH_SIZE = 128 MiB and WRITE_SIZE = 256 MiB.
 # Summaries: profiles/gemv_k_gemv8_k_sweep_m1-16_k5120.md,
-# profiles/k_gemm_dit_attention_m8192_k5120.md, profiles/hbm_counters_copy_256MiB.md.
+# profiles/k_gemm256_k_wfrag_dit_shapes.md, profiles/hbm_counters_copy_256MiB.md.
 # Re-measure when the kernels change.
 TRAFFIC_GEMV_MEAN = 33641612        # mean over the six GEMV shapes (algorithmic mean 32899072)
-TRAFFIC_GEMM = {"attn_qkv": 2324594574, "attn_out": 703181960}
+TRAFFIC_GEMM = {"attn_qkv": 2645679488, "attn_out": 907092864}  # k_wfrag + k_gemm256
 
 
 def q4k_bytes(N, K):
@@ -802,8 +802,8 @@ def main():
     ach = sum_flop / (sum_t * 1e-3)
     roofline_gemm = {"bound": "mfma", "achieved": round(ach / 1e12, 1), "peak": MFMA_F16_PEAK / 1e12,
                      "unit": "TFLOP/s", "frac": round(ach / MFMA_F16_PEAK, 4),
-                     "traffic": TRAFFIC_GEMM["attn_qkv"], "traffic_kernel": "k_gemm attn_qkv M=8192 N=15360",
-                     "kernel": "k_gemm (fh3_hip_matmul_prepared_dev, n_tok>64)",
+                     "traffic": TRAFFIC_GEMM["attn_qkv"], "traffic_kernel": "k_wfrag + k_gemm256 attn_qkv M=8192 N=15360",
+                     "kernel": "k_wfrag + k_gemm256 (fh3_hip_matmul_prepared_dev, n_tok>=1024)",
                      "note": "2*M*N*K per launch over launch time, summed over the DiT GEMMs; "
                              "fp16 operands, fp32 accumulation; peak is dense fp16 MFMA"}
     extra["dit_gemms"] = gemms

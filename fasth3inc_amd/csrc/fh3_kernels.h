@@ -123,8 +123,8 @@ hipError_t fh3k_gemm256(int type, const void *W, int64_t row_bytes, int N, int K
                         const float *xs_inv, const float *bias, float *y, int M, int epi, const float *aux,
                         void *wfrag, hipStream_t st);
 size_t fh3k_gemm256_bytes(int type, int N, int K, int M, int epi);
-// Prepared rows k_gemm reads for M tokens (its tiles cover 128 or 256
-// tokens; at most round_up(M, fh3k_gemm_row_pad())).
+// Prepared rows the tiles read for M tokens (k_gemm's cover 128 or 256 tokens,
+// k_gemm256's 256; at most round_up(M, fh3k_gemm_row_pad())).
 int fh3k_gemm_rows(int M);
 
 // Middle M (1 <= M <= fh3k_midm_max_tokens()): K split into S windows, partial

@@ -2388,11 +2388,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *__restrict__ W, 
 // The MFMAs are written as asm with the accumulator tied (the builtin's separate
 // destination made the compiler move accumulators between registers, +10 % at
 // K = 5120) and sched_barrier keeps the loads where they stand.
-// Dequantising inside this kernel instead (78 VALU per 64 MFMAs) measured 0.72
-// against 0.54 us per stage: with one wavefront per SIMD the VALU does not
-// overlap with the MFMAs.
-// K = 13824, N = 5120, 32768 tokens: 4102 us (k_gemm) -> 3262 + 30 us
-// (1.42 PFLOP/s); K = 5120, N = 15360, 8192 tokens: 1177 -> 960 + 32 us.
+// Dequantising inside this kernel instead costs 78 VALU per 64 MFMAs, which one
+// wavefront per SIMD does not overlap with them; decoding once costs one pass.
+// K = 13824, N = 5120, 32768 tokens: 4102 us (k_gemm) -> 3232 + 40 us (1.44
+// PFLOP/s: 0.75 us a stage, the matrix pipe 81 % busy at 1.67 GHz); K = 5120, N =
+// 15360, 8192 tokens: 1177 -> 970-1020 + 38 us (70 % at 1.80 GHz).
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
 constexpr int G256_B = 256;  // tokens and weight rows of a tile
@@ -3752,7 +3752,7 @@ extern "C" hipError_t fh3k_midm_epi(const void *W, int64_t row_bytes, int N, int
 // workgroup (~5 us): rounds of 512 resident workgroups x (C + 1), plus the
 // partial sums (written and read: S*M*N*8 bytes at ~5 TB/s) and the extra
 // launch.
-// 32-token blocks per k_gemm wavefront: one (128-token tiles) up to 128
+// 32-token blocks per k_gemm wavefront (k_gemm256 has tiles of its own): one (128-token tiles) up to 128
 // tokens, and up to 256 while the 128-token tiles number at most 128; two
 // (256-token tiles) otherwise.  (Measured, K = 5120, calls incl. preparation
 // and ordered sum: at N = 5120, 65-128 tokens 26.2-28.4 us against 32.2-34.3

@@ -18,7 +18,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // fragments are made here (k_xprep_any's scale rule and rounding) and shared
 // through LDS.  The same products in the same k order as k_gemm16, so the same
 // bits.  2880 x 96 -> 5376 with its bias: 43.5 -> 17.3 us per call (3.7 TB/s),
-// 16384 tokens 191 -> 82, 100 tokens 29.9 -> 5.8, one token 10.2 -> 5.1.
+// 16384 tokens 191 -> 82, 100 tokens 29.9 -> 5.8, one token 10.2 -> 5.1 (K = 96).
+// y must not lie over x.
 constexpr int SHORT_K = 128, SHORT_M = 128, SHORT_N = 128;
 __global__ __launch_bounds__(256) void k_short16(const _Float16 *__restrict__ W16, int N, int K,
                                                  const float *__restrict__ X, const float *__restrict__ bias,

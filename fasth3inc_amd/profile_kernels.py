@@ -10,11 +10,12 @@ Workloads (each launch sequence is preceded by one untimed warmup launch):
          (M = 16, after k_xprep), weights rotated over more than 256 MB of
          device copies so they come from HBM
   gemm   the DiT attention shapes (M=8192, K=5120, N in {15360,5120}):
-         fh3_hip_matmul_prepared_dev -> k_gemm, and the activation prep k_xprep
+         fh3_hip_matmul_prepared_dev -> k_wfrag, k_gemm256, and the activation
+         prep k_xprep_r8
   mlp    the DiT MLP shapes (M=32768: up and gate K=5120 -> N=13824 with a
          2-decade per-super-block scale spread, down K=13824 -> N=5120 on
-         SiLU-gated activations): fh3_hip_matmul_prepared_dev -> k_gemm, and
-         the activation prep k_xprep_r8
+         SiLU-gated activations): fh3_hip_matmul_prepared_dev -> k_wfrag,
+         k_gemm256, and the activation prep k_xprep_r8
   te     the text encoder's long Q4_K rows at M = 1 and 16 (o-projection
          K=8192 -> N=5120, down-projection K=25600 -> N=5120):
          fh3_hip_matmul_prepared_dev -> k_gemv8 (M = 1, K = 8192) or k_sweep in

@@ -78,7 +78,11 @@ int fh3_hip_dequant_dev(int type, const void *d_src, float *d_dst, int64_t rows,
  * n_tok * in * 2 bytes, plus S * n_tok * out * 4 bytes of partial sums where
  * K is split (the FH3_HIP_PATH_MIDM path, S <= in / 512; the GEMM path when
  * its 256 x 128 tiles number fewer than about 512, S <= in / 512 and
- * S * tiles <= 4096); calls that overlap on different streams race on it.  Q4_K, Q5_K and Q6_K products of more than 64
+ * S * tiles <= 4096); calls that overlap on different streams race on it.  F16
+ * rows of at most 128 values (in % 8 == 0) use none, unless d_y lies over d_x.
+ * Q4_K, Q5_K and Q6_K products of 1024 tokens and more may also decode their
+ * weights into library memory of their own (fh3_hip_matmul_workspace_bytes);
+ * no call races on that.  Q4_K, Q5_K and Q6_K products of more than 64
  * tokens need out * row_bytes < 2^32 (32-bit row offsets; 7.6e9 Q4_K weights). */
 int fh3_hip_matmul_dev(const Fh3W *w, const float *d_x, float *d_y, int n_tok,
                        const float *d_bias_or_null, void *stream);
@@ -92,12 +96,14 @@ int fh3_hip_matmul_dev(const Fh3W *w, const float *d_x, float *d_y, int n_tok,
  *     rows of whole super-blocks one fp32 sum per 32-value group);
  *   fh3_hip_prepare_x_dev: fill d_prep (16-byte aligned) from d_x[n_tok][in];
  *   fh3_hip_matmul_prepared_dev: the product from a prepared buffer; same
- *     results as fh3_hip_matmul_dev.  Its only library workspace is the
+ *     results as fh3_hip_matmul_dev.  Its library workspace is the
  *     partial sums of the split-K kernels: the FH3_HIP_PATH_MIDM path, and
  *     the FH3_HIP_PATH_GEMM path while its 256 x 128 tiles number fewer than
  *     about 512 (roughly 65..2048 tokens; fh3_hip_matmul_workspace_bytes
  *     gives the exact size).  Weights of a type other than Q4_K also use the
- *     fp16-row buffer.  (For the FH3_HIP_PATH_GEMV8 shapes the prepared form
+ *     fp16-row buffer (Q5_K and Q6_K of whole super-blocks do not), and
+ *     products of 1024 tokens and more that do not split K may decode their
+ *     weights into library memory (see there).  (For the FH3_HIP_PATH_GEMV8 shapes the prepared form
  *     is a copy of x; it is valid only while fh3_hip_set_path keeps the
  *     setting it was prepared under.  The fragment form, with its group sums,
  *     is valid under any setting.) */
@@ -224,20 +230,26 @@ int fh3_hip_graph_destroy(void *graph_exec);
 
 /* Bytes of library workspace a product allocates (0 when none): the prepared
  * activations of fh3_hip_matmul_dev / fh3_hip_matmul_epi_dev (prepared = 0)
- * plus the partial sums of the split-K kernels; with prepared = 1 the same for
- * fh3_hip_matmul_prepared_dev / _prepared_epi_dev.  epi as below.  Under the
- * current fh3_hip_set_path setting.  Not counted: the fp16 weights (out * in *
- * 2 bytes, at most 1 GiB) that a Q4_K, Q5_K or Q6_K product of about 1024
- * tokens or more decodes when it can.  One buffer, kept until
- * fh3_hip_shutdown, serves all streams (their products wait for one another on
- * the device); under capture, and where the memory is not to be had, the
- * weights are read in place instead, with the same results. */
+ * plus the partial sums of the split-K kernels and the fp16 rows of other weight
+ * types; with prepared = 1 the same for fh3_hip_matmul_prepared_dev /
+ * _prepared_epi_dev.  epi as below.  Under the current fh3_hip_set_path setting.
+ * An upper bound for F16 rows of at most 128 values (fh3_hip_matmul_dev).
+ * Not counted: the fp16 weights (out, rounded up to 256 rows, * in * 2 bytes, at
+ * most 1 GiB) that a Q4_K, Q5_K or Q6_K product of 1024 tokens or more decodes
+ * where that is faster.  They stand in at most two buffers, one to a stream, and
+ * take at most an eighth of the memory that is free at the time; kept for the
+ * next such product, they go back when an allocation of the library finds no
+ * memory left, and in fh3_hip_shutdown.  Under capture, while both buffers are
+ * at work for other streams, and where the memory is not to be had, the
+ * weights are read in place instead, with the same results: no stream waits
+ * for another, and no call fails for this memory. */
 size_t fh3_hip_matmul_workspace_bytes(const Fh3W *w, int n_tok, int epi, int prepared);
 
 /* The no-allocation product, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc).  Same arguments, kernels and bit-identical results as
- * fh3_hip_matmul_dev with Q4_K weights and no epilogue, but its workspace is
+ * hipMalloc).  Same arguments and bit-identical results as
+ * fh3_hip_matmul_dev with Q4_K weights and no epilogue, and the same kernels but
+ * that weights are always read in place; its workspace is
  * a fixed array of FH3_HIP_NOALLOC_SCRATCH_BYTES in device memory that the
  * library binds in fh3_hip_init (each device holds its own copy until the
  * process ends).  The call allocates and frees nothing; it returns
